@@ -18,10 +18,13 @@
 // enables split-K (qh_gemm_e4m3 / qh_gemm_e4m3_grouped).  The reference entry
 // point fp8_gemm_batch passes none and never splits.
 //
-// Two kernels, both with a 2 x 2 grid of waves per output tile in an
-// XCD-aware tile order (the row tiles of one weight tile run on one XCD and
-// share it in that XCD's L2):
-//  - gemm_dma_kernel (every launch whose operands it can take): persistent
+// Three kernels, all in an XCD-aware tile order (the tiles that run on one XCD
+// share rows of X and of W in that XCD's L2):
+//  - gemm_tile_kernel (gemm_tile.h; block scales): one output tile per
+//    workgroup, from 16 x 16 with K shared out over eight waves (a few rows) to
+//    128 x 320 (thousands), the shape picked by a time model (gemm_plan);
+//  - gemm_dma_kernel (other scale modes, and where the model favours it):
+//    a 2 x 2 grid of waves per tile; persistent
 //    workgroups stream (tile or tile K slice, K block) units through a
 //    two-stage LDS ring filled by direct-to-LDS loads, on 64 x 64 tiles
 //    (three workgroups per CU), 64 x 128 (two) or 128 x 192 (one), the plan
@@ -34,6 +37,7 @@
 // Operand layout of the 32x32x16 bf16 instruction (measured on gfx950):
 // lane l holds A[l % 32][8 (l / 32) + r] and B[8 (l / 32) + r][l % 32],
 // r = 0..7, and accumulator value e is C[8 (e / 4) + 4 (l / 32) + e % 4][l % 32].
+#include "gemm_tile.h"
 #include "qh_common.h"
 #include "qh_gemm.h"
 #include "qh_norm.h"
@@ -816,6 +820,105 @@ __global__ __launch_bounds__(256) void splitk_add_rmsnorm_kernel(const float* pa
   }
 }
 
+// ---- tile kernel: one output tile per workgroup (gemm_tile.h) -----------------
+// Workgroup b runs on XCD b % 8.  XCD x takes the x-th eighth of the items, in
+// an order of gm row tiles at a time (row tile fastest), so the items running
+// on an XCD share a few row tiles of X and of W in its L2.  With 8 K slices
+// each XCD takes one slice of every tile instead: it then reads an eighth of
+// X and of W.
+template <typename C, typename ScaleT, bool SPLIT>
+__global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(const uint16_t* x, GemmGroup g, int M, int K,
+                                                                  int nstep, int tiles_n, int tiles_m, int S_arg,
+                                                                  float* part, int ldp, int gm) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  const int S = SPLIT ? S_arg : 1;
+  const int xc = (int)blockIdx.x & 7, b = (int)blockIdx.x >> 3;
+  const int T = tiles_m * tiles_n;
+  int item = b, z = xc;
+  if (!(SPLIT && S == 8)) {
+    const int per = (T * S + 7) / 8;
+    if (b >= per) return;
+    item = xc * per + b;
+    z = SPLIT ? item % S : 0;
+    if (SPLIT) item /= S;
+  }
+  if (item >= T) return;
+  const int grp = item / (gm * tiles_n), rr = item - grp * gm * tiles_n;
+  const int gme = min(gm, tiles_m - grp * gm);
+  const int tn = rr / gme, m0 = (grp * gm + rr % gme) * C::BM;
+  int si = 0;
+#pragma unroll
+  for (int t = 1; t < 4; ++t)
+    if (t < g.nseg && tn >= g.tstart[t]) si = t;
+  const int N = g.N[si], n0 = (tn - g.tstart[si]) * nstep;
+  const int U = K / C::KU;
+  qh_tile::Work t;
+  t.x = x + (size_t)m0 * K;
+  t.w = g.w[si] + (size_t)n0 * K;
+  t.rows_m = min(M - m0, C::BM);
+  t.rows_n = min(N - n0, nstep);
+  t.K = K;
+  t.u0 = SPLIT ? (int)((long)U * z / S) : 0;
+  t.u1 = SPLIT ? (int)((long)U * (z + 1) / S) : U;
+  t.s = g.s[si];
+  t.kb = g.kb[si];
+  t.n0 = n0;
+  t.nblk_last = (N - 1) >> 7;
+  f32x4 acc[C::MI][C::NJ];
+  qh_tile::mainloop<C, ScaleT>(t, smem, acc);
+  if (SPLIT) {
+    float* pz = part + ((size_t)z * M + m0) * ldp + (size_t)tn * nstep;
+    qh_tile::finish<C>(t, smem, acc, [&](int m, int n, f32x4 v) { *(f32x4*)(pz + (size_t)m * ldp + n) = v; });
+  } else {
+    uint16_t* y = g.y[si] + (size_t)m0 * N + n0;
+    const bool vec = N % 4 == 0 && (uintptr_t)g.y[si] % 8 == 0;
+    qh_tile::finish<C>(t, smem, acc, [&](int m, int n, f32x4 v) {
+      uint16_t* dst = y + (size_t)m * N + n;
+      if (vec) {
+        *(u32x2*)dst = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+      } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (n + c < t.rows_n) dst[c] = f2bf(v[c]);
+      }
+    });
+  }
+}
+
+// tiles_n tiles of nstep columns over all segments; reduce as launch_gemm_dma.
+template <typename C, typename ScaleT, bool CAN_SPLIT>
+void launch_gemm_tile(const uint16_t* x, const QhGemmSeg* seg, int nseg, int M, int K, hipStream_t st, int nstep,
+                      int S, float* part, bool reduce) {
+  GemmGroup g = {};
+  g.nseg = nseg;
+  int tiles_n = 0;
+  for (int t = 0; t < nseg; ++t) {
+    g.w[t] = (const uint8_t*)seg[t].w;
+    g.s[t] = seg[t].s;
+    g.y[t] = (uint16_t*)seg[t].y;
+    g.N[t] = seg[t].N;
+    g.kb[t] = seg[t].kb;
+    g.tstart[t] = tiles_n;
+    tiles_n += (seg[t].N + nstep - 1) / nstep;
+  }
+  const int tiles_m = (M + C::BM - 1) / C::BM, ldp = tiles_n * nstep;
+  const long T = (long)tiles_m * tiles_n;
+  const int gm = (int)min((long)tiles_m, 4L);
+  if constexpr (CAN_SPLIT) if (S > 1) {
+    const unsigned grid = S == 8 ? 8 * T : 8 * ((T * S + 7) / 8);
+    hipLaunchKernelGGL((gemm_tile_kernel<C, ScaleT, true>), dim3(grid), dim3(C::THREADS), (size_t)C::LDS, st, x, g, M,
+                       K, nstep, tiles_n, tiles_m, S, part, ldp, gm);
+    if (reduce) {
+      const size_t quads = (size_t)M * ldp / 4;
+      hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st,
+                         (const float*)part, S, M, ldp, g, nstep);
+    }
+    return;
+  }
+  hipLaunchKernelGGL((gemm_tile_kernel<C, ScaleT, false>), dim3((unsigned)(8 * ((T + 7) / 8))), dim3(C::THREADS),
+                     (size_t)C::LDS, st, x, g, M, K, nstep, tiles_n, tiles_m, 1, (float*)nullptr, ldp, gm);
+}
+
 template <int BN>
 GemmGroup make_group(const QhGemmSeg* seg, int nseg, int& tiles_n) {
   GemmGroup g = {};
@@ -875,17 +978,124 @@ void launch_gemm_small(const uint16_t* x, const QhGemmSeg* seg, int nseg, int M,
 constexpr size_t kSplitPartBytes = (size_t)1024 * 64 * 64 * sizeof(float);
 
 namespace {
-// Launch plan of the ring kernel: tile shape, workgroups per CU, K slices.
+// Launch plan: a shape of the tile kernel (tile >= 0: index into kTiles, nstep
+// columns per tile) or of the ring kernel (tile = -1: bm x bn tiles, wpc
+// workgroups per CU), and the K slices S.  ldp: row stride of the partials.
 struct GemmPlan {
-  int bm, bn, wpc, S;
+  int tile, bm, bn, wpc, nstep, S, ldp;
 };
 
-// Cycles one workgroup spends per (tile, 128-wide K block) unit at its
-// occupancy (64 x 64: three workgroups per CU, 64 x 128: two, 128 x 192:
-// one), measured on MI355X at M = 512 (X fits the XCD's L2) and at M = 3700
-// (grouped row tiles; X streams): 2.0 / 2.2 / 4.3 and 2.5 / 2.6 / 3.8
-// thousand.  (128 x 128 tiles, 3.0 / 2.8 thousand, were never the fastest
-// plan for a prefill shape.)
+// Tile kernel shapes: MI, NJ, WM, WN, KG, KU, DS (gemm_tile.h) and whether they
+// are built for split-K.
+#define QH_TILE_SHAPES(V)             \
+  V(0, 1, 1, 1, 1, 8, 64, 3, false)   \
+  V(1, 1, 3, 1, 1, 8, 64, 3, false)   \
+  V(2, 2, 2, 1, 1, 8, 64, 2, false)   \
+  V(3, 2, 3, 1, 1, 8, 64, 2, true)    \
+  V(4, 4, 3, 1, 1, 4, 64, 3, true)    \
+  V(5, 1, 5, 2, 2, 2, 128, 2, true)   \
+  V(6, 2, 5, 2, 2, 2, 128, 2, true)   \
+  V(7, 2, 5, 4, 2, 1, 128, 2, true)   \
+  V(8, 4, 4, 2, 4, 1, 128, 2, false)  \
+  V(9, 4, 5, 2, 4, 1, 64, 4, false)
+
+// Time model of a launch, in us: a + b (rounds x passes) + c rounds + d (MB a
+// CU pulls in), rounds = ceil(tiles / CUs), passes = K units of one K group.
+// Fitted to 26 row counts (2 .. 3700) x 11 (N, K) (512 x 256 .. 18432 x 2560) on
+// MI355X with the weights out of the caches, rms error 5 - 14 %; over those
+// 286 shapes the plan it picks is 2 % slower than the fastest shape measured.
+struct TileShape {
+  int bm, bn, kg, ku;
+  bool split;
+  double a, b, c, d;
+};
+#define QH_BM(MI, WM) 16 * MI * WM
+#define QH_V(id, MI, NJ, WM, WN, KG, KU, DS, SP) {QH_BM(MI, WM), QH_BM(NJ, WN), KG, KU, SP, QH_TIME_##id},
+#define QH_TIME_0 2.074, 0.2978, 0.9993, 0.5571
+#define QH_TIME_1 0.8717, 0.2865, 2.862, 9.224
+#define QH_TIME_2 0.8305, 0.2711, 2.552, 6.744
+#define QH_TIME_3 0.6686, 0.2669, 3.074, 8.796
+#define QH_TIME_4 1.577, 0.5643, 2.84, 0.6752
+#define QH_TIME_5 0.0, 0.8451, 3.447, 5.105
+#define QH_TIME_6 1.093, 1.245, 3.126, 2.955
+#define QH_TIME_7 0.0, 1.121, 3.915, 2.799
+#define QH_TIME_8 0.0, 1.431, 4.599, 4.072
+#define QH_TIME_9 0.0, 1.113, 5.439, 3.584
+constexpr TileShape kTiles[] = {QH_TILE_SHAPES(QH_V)};
+#undef QH_V
+
+inline long tiles_of(const QhGemmSeg* seg, int nseg, int bn) {
+  long n = 0;
+  for (int t = 0; t < nseg; ++t) n += (seg[t].N + bn - 1) / bn;
+  return n;
+}
+
+// The plan with the shortest modelled time.
+//  - Tile kernel: 128 x 128 block scales, up to 128 K blocks (the scales of a
+//    tile stay in registers).  Tiles narrower than the shape's when they all
+//    run at once: the CUs then share the weight bytes evenly (2560 x 9216, 24
+//    rows: 13.9 us with 16 columns, 13.2 with 12).
+//  - Split K (caller workspace only): the partials' round trip and the
+//    finishing launch; a lone segment is an output projection, whose finish
+//    replaces the add + norm launch that would follow.
+//  - Ring kernel beside it where its model holds and the tile shapes leave
+//    CUs idle: one 64 x 64 tile per CU (1024 x 1024 x 2560: 15.4 us against
+//    17.9), one round of 64 x 128 at two workgroups per CU (400 x 8192 x 2560:
+//    27.3 against 30.4).  Every other ring plan lost (3700 x 18432 x 2560: 387
+//    against 346 us; 24 x 2560 x 9216: 48 against 12).
+//  - Other scale modes: the ring kernel's own plans (gemm_plan_ring).
+GemmPlan gemm_plan_ring(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const void* ws, size_t ws_bytes);
+
+GemmPlan gemm_plan(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const void* ws, size_t ws_bytes) {
+  const int KB = K / 128;
+  long nsum = 0;
+  bool block = KB >= 2 && KB <= 128;
+  for (int t = 0; t < nseg; ++t) {
+    block = block && seg[t].kb == KB;
+    nsum += seg[t].N;
+  }
+  if (!block) return gemm_plan_ring(M, K, seg, nseg, cus, ws, ws_bytes);
+  GemmPlan best = {-1, 64, 64, 3, 64, 1, 0};
+  double best_t = 1e300;
+  const long r64 = (long)((M + 63) / 64) * tiles_of(seg, nseg, 64), r128 = (long)((M + 63) / 64) * tiles_of(seg, nseg, 128);
+  if (r64 <= cus) best_t = 2.8 + 0.61 * KB;
+  if (r128 > cus && r128 <= 2L * cus && 5.39 + 1.06 * KB < best_t) {
+    best_t = 5.39 + 1.06 * KB;
+    best = {-1, 64, 128, 2, 128, 1, 0};
+  }
+  for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
+    const TileShape& c = kTiles[i];
+    const long tiles_m = (M + c.bm - 1) / c.bm;
+    for (int S = 1; S <= 8; S *= 2) {
+      int nstep = c.bn;
+      long tiles_n = tiles_of(seg, nseg, nstep);
+      if (S > 1) {
+        if (!c.split || !ws || KB % S != 0 || (size_t)S * M * tiles_n * nstep * sizeof(float) > ws_bytes) continue;
+      } else if (tiles_m * tiles_n <= cus) {
+        nstep = (int)min((long)c.bn, (nsum * tiles_m / cus + 3) / 4 * 4);
+        nstep = nstep < 4 ? 4 : nstep;
+        while (nstep < c.bn && tiles_m * tiles_of(seg, nseg, nstep) > cus) nstep += 4;
+        tiles_n = tiles_of(seg, nseg, nstep);
+      }
+      const long rounds = (tiles_m * tiles_n * S + cus - 1) / cus;
+      const int units = (K / c.ku + S - 1) / S, passes = (units + c.kg - 1) / c.kg;
+      const double mb = (double)rounds * (2.0 * min(M, c.bm) + nstep) * K / S * 1e-6;
+      double t = c.a + c.b * (double)rounds * passes + c.c * (double)rounds + c.d * mb;
+      if (S > 1) t += (nseg == 1 ? 1.0 : 3.0) + (S + 0.5) * M * (double)tiles_n * nstep * 1e-6;
+      if (t < best_t * 0.99) {
+        best_t = t;
+        best = {i, c.bm, c.bn, 1, nstep, S, (int)(tiles_n * nstep)};
+      }
+    }
+  }
+  return best;
+}
+
+// Cycles one workgroup of the ring kernel spends per (tile, 128-wide K block)
+// unit at its occupancy (64 x 64: three workgroups per CU, 64 x 128: two,
+// 128 x 192: one), measured on MI355X at M = 512 (X fits the XCD's L2) and at
+// M = 3700 (grouped row tiles; X streams): 2.0 / 2.2 / 4.3 and 2.5 / 2.6 / 3.8
+// thousand.
 struct GemmShape {
   int bm, bn, wpc;
   double cycles_small, cycles_large;
@@ -893,20 +1103,16 @@ struct GemmShape {
 constexpr GemmShape kGemmShapes[] = {{64, 64, 3, 2030.0, 2460.0}, {64, 128, 2, 2200.0, 2600.0},
                                      {128, 192, 1, 4280.0, 3760.0}};
 
-// The plan with the shortest modelled time: units on the busiest XCD's
-// busiest workgroup times the unit cost, plus, when K is split (caller
+// The ring kernel's plan with the shortest modelled time: units on the busiest
+// XCD's busiest workgroup times the unit cost, plus, when K is split (caller
 // workspace only, 2 .. 8 slices of >= 4 K blocks each), the partials'
-// round trip through memory and the finishing launch (≈ 6 us: 128 x 10240 x
-// 2560 took 17.7 us unsplit and 21.9 us in two slices).  Deeper rings for
-// 64 x 64 tiles (three or four stages, fewer workgroups per CU) measured no
-// faster at M = 128 and 512.
-GemmPlan gemm_plan(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const void* ws, size_t ws_bytes) {
+// round trip through memory and the finishing launch (≈ 6 us).
+GemmPlan gemm_plan_ring(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const void* ws, size_t ws_bytes) {
   const int KB = K / 128;
-  GemmPlan best = {64, 64, 3, 1};
+  GemmPlan best = {-1, 64, 64, 3, 64, 1, 0};
   double best_t = 1e300;
   for (const GemmShape& c : kGemmShapes) {
-    long tiles_n = 0;
-    for (int t = 0; t < nseg; ++t) tiles_n += (seg[t].N + c.bn - 1) / c.bn;
+    const long tiles_n = tiles_of(seg, nseg, c.bn);
     const long tiles_m = (M + c.bm - 1) / c.bm;
     const long slots = (long)cus * c.wpc / 8;  // workgroups per XCD
     for (int S = 1; S <= 8; ++S) {
@@ -919,7 +1125,7 @@ GemmPlan gemm_plan(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const 
       if (S > 1) t += (double)S * M * tiles_n * c.bn * 4.0 * 2.0 / 2048.0 + 13000.0;
       if (t < best_t * 0.98) {
         best_t = t;
-        best = {c.bm, c.bn, c.wpc, S};
+        best = {-1, c.bm, c.bn, c.wpc, c.bn, S, (int)(tiles_n * c.bn)};
       }
     }
   }
@@ -929,6 +1135,16 @@ GemmPlan gemm_plan(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const 
 template <typename ScaleT>
 void launch_gemm_plan(const GemmPlan& pl, const uint16_t* x, const QhGemmSeg* seg, int nseg, int M, int K,
                       hipStream_t st, int cus, float* part, bool reduce) {
+  switch (pl.tile) {
+#define QH_V(id, MI, NJ, WM, WN, KG, KU, DS, SP)                                                                     \
+  case id:                                                                                                           \
+    launch_gemm_tile<qh_tile::Cfg<MI, NJ, WM, WN, KG, KU, DS>, ScaleT, SP>(x, seg, nseg, M, K, st, pl.nstep, pl.S,  \
+                                                                           part, reduce);                            \
+    return;
+    QH_TILE_SHAPES(QH_V)
+#undef QH_V
+    default: break;
+  }
   if (pl.bm == 128)
     launch_gemm_dma<ScaleT, 2, 192, 128>(x, seg, nseg, M, K, st, cus, pl.wpc, pl.S, part, reduce);
   else if (pl.bn == 128)
@@ -1031,7 +1247,7 @@ int qh_launch_gemm_e4m3_add_rmsnorm(const void* x, const void* w, const void* s,
       float* part = (float*)ws;
       if (scale_bf16) launch_gemm_plan<uint16_t>(pl, (const uint16_t*)x, &seg, 1, M, K, st, cus, part, false);
       else launch_gemm_plan<float>(pl, (const uint16_t*)x, &seg, 1, M, K, st, cus, part, false);
-      const int S = pl.S, ldp = ((N + pl.bn - 1) / pl.bn) * pl.bn;
+      const int S = pl.S, ldp = pl.ldp;
       const int v = (N / 8 + 255) / 256;
 #define QH_SAN(V, SC)                                                                                          \
   hipLaunchKernelGGL((splitk_add_rmsnorm_kernel<V, SC>), dim3(M), dim3(256), 0, st, (const float*)part, S, M, ldp, N, \

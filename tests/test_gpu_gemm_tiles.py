@@ -1,0 +1,96 @@
+"""The prefill GEMM's tile shapes against the product in 64 bits (MI355X only)."""
+import pytest
+import torch
+
+from oracle import qwen35_oracle as orc
+from qwen35_amd import abi, ops
+
+from _util import bf, gen, quant, randn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def product(x, w, s):
+    """(X deq(W)^T, |X| |deq(W)|^T) in 64 bits."""
+    d = orc.dequant(w, s.float()).to(DEV).double()
+    x = x.to(DEV).double()
+    return x @ d.t(), x.abs() @ d.abs().t()
+
+
+def check(y, ref, mag, K, what):
+    """bf16 rounding of the result (8 significant bits: at most 2^-8 of it) and K fp32 additions of products
+    whose magnitudes add up to mag (each at most 2^-24 of a partial sum <= mag)."""
+    err = (y.double() - ref).abs()
+    bound = ref.abs() * 2.0 ** -8 + mag * (K * 2.0 ** -24) + 1e-38
+    bad = err > bound
+    assert torch.isfinite(y.float()).all() and not bad.any(), \
+        f"{what}: {int(bad.sum())} of {bad.numel()} off, worst {float((err / bound).max()):.2f} of the bound"
+
+
+# The shape that 256 CUs take for each (rows x columns of the tile, waves along K), at row and
+# column counts that leave ragged last tiles; K is as short as the shape's choice allows, so that
+# K groups with no unit of their own and rings longer than K are among them.
+@pytest.mark.parametrize("M,N,K", [
+    (2, 4, 256), (9, 5, 640), (16, 2560, 9216), (17, 33, 256),          # 16 x 16, 8 waves
+    (2, 8544, 384), (3, 8217, 640), (16, 9999, 2560),                   # 16 x 48, 8 waves
+    (2, 4185, 256), (31, 2561, 4096), (65, 1673, 256),                  # 32 x 32, 8 waves
+    (2, 9301, 896), (29, 9030, 512), (72, 2827, 384),                   # 32 x 48, 8 waves
+    (33, 6549, 768), (91, 4315, 896), (131, 2522, 768),                 # 64 x 48, 4 waves
+    (2, 16557, 256), (23, 16850, 640), (271, 2523, 1024),               # 32 x 160, 2 groups
+    (71, 15113, 256), (866, 1779, 256), (129, 9217, 1536),              # 64 x 160, 2 groups
+    (137, 13615, 256), (635, 4513, 256), (2490, 1595, 384),             # 128 x 160
+    (281, 13694, 256), (815, 7373, 512),                                # 128 x 256
+    (391, 18067, 256), (943, 8514, 384),                                # 128 x 320
+    (5, 300, 16384), (5, 300, 16512),                                   # 128 K blocks, and one more (ring kernel)
+])
+def test_gemm_tile_shapes(M, N, K):
+    g = gen(M * 3 + N + K)
+    w, s = quant(g, N, K)
+    s = s * (1.0 + torch.rand(s.shape, generator=g))   # scales that differ from block to block
+    s[-1, -1] = 0.0                                    # and an empty block
+    x = bf(randn(g, M, K))
+    for scale in (s, s.to(torch.bfloat16)):            # bf16: fp8_gemm_batch
+        ref, mag = product(x, w, scale)
+        y = ops.fp8_linear(x.to(DEV), w.to(DEV), scale.to(DEV))
+        check(y, ref, mag, K, f"{M} x {N} x {K} {scale.dtype}")
+
+
+@pytest.mark.parametrize("M,N,K", [(24, 2560, 9216), (128, 2560, 9216), (100, 2500, 4096), (300, 2560, 2560),
+                                   (512, 2560, 9216), (2, 12563, 1024), (37, 1001, 9216)])
+def test_gemm_tile_split_k(M, N, K):
+    """K slices over workgroups (a workspace given), plain and fused with the residual add."""
+    g = gen(M + N + K)
+    w, s = quant(g, N, K)
+    x, h = bf(randn(g, M, K)).to(DEV), bf(randn(g, M, N)).to(DEV)
+    lib = abi.load()
+    dw, ds = w.to(DEV), s.to(DEV)
+    ws = torch.full((int(lib.qh_gemm_workspace_size(M, K)),), 0xFF, dtype=torch.uint8, device=DEV)  # NaN partials
+    y, o = torch.empty(2, M, N, dtype=torch.bfloat16, device=DEV).unbind(0)
+    abi.check(lib.qh_gemm_e4m3(abi.ptr(x), abi.ptr(dw), abi.ptr(ds), abi.ptr(y), M, N, K, K // 128, 0, abi.ptr(ws),
+                               ws.numel(), abi.stream_handle()), "gemm")
+    ref, mag = product(x, w, s)
+    check(y, ref, mag, K, "workspace")
+    h2 = h.clone()
+    abi.check(lib.qh_gemm_e4m3_add_rmsnorm(abi.ptr(x), abi.ptr(dw), abi.ptr(ds), abi.ptr(o), M, N, K, K // 128, 0,
+                                           abi.ptr(h2), None, None, 1e-6, abi.ptr(ws), ws.numel(),
+                                           abi.stream_handle()), "gemm_add")
+    assert torch.equal(h2, (h.float() + y.float()).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M", [3, 20, 128, 700])
+def test_gemm_tile_segments(M):
+    """Segments of unequal width, one of them a few columns, each with its own scales."""
+    K, ns = 1024, (1000, 8192, 32, 5)
+    g = gen(M)
+    x = bf(randn(g, M, K))
+    dx, lib = x.to(DEV), abi.load()
+    segs = [quant(g, n, K) for n in ns]
+    ys = [torch.empty(M, n, dtype=torch.bfloat16, device=DEV) for n in ns]
+    keep, args = [], []
+    for (w, s), y, n in zip(segs, ys, ns):
+        keep += [w.to(DEV), s.to(DEV)]
+        args += [abi.ptr(keep[-2]), abi.ptr(keep[-1]), abi.ptr(y), n, K // 128]
+    abi.check(lib.qh_gemm_e4m3_grouped(abi.ptr(dx), M, K, 4, *args, 0, None, 0, abi.stream_handle()), "grouped")
+    for (w, s), y, n in zip(segs, ys, ns):
+        check(y, *product(x, w, s), K, f"{M} rows, {n} columns")
