@@ -244,6 +244,14 @@ int qh_lm_head_argmax(const void* x, const float* norm_w, float eps, int K, cons
                       int64_t* tok_hist, int hist_len, int* pos_dev, const void* embed,
                       void* embed_out, qh_stream_t stream);
 
+/* lm_head over M rows of hidden states (F.linear with logits_to_keep != 1,
+ * main.py:1596-1604): xn (bf16 [M, K] scratch, distinct from x) = the (1+w)
+ * RMSNorm of x's rows, logits (bf16 [M, N]) = bf16(xn . w^T); norm_w null: x is
+ * used as it is and xn may be null.  K % 64 == 0, x, xn and w 16-byte aligned.
+ * No counterpart in the reference, which calls F.linear. */
+int qh_lm_head_rows(const void* x, const float* norm_w, float eps, int M, int K, const void* w, int N,
+                    void* xn, void* logits, qh_stream_t stream);
+
 /* Workspace bytes for qh_sample_top_p over a V-entry vocabulary. */
 size_t qh_sample_workspace_size(int V);
 

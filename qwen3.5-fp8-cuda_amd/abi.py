@@ -77,6 +77,7 @@ NATIVE_SIGNATURES = {
     "qh_lm_head_scratch_bytes": (_sz, [_i]),
     "qh_lm_head_argmax": (_i, [_vp, _vp, _f, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _i,
                                _vp, _vp, _vp, _vp]),
+    "qh_lm_head_rows": (_i, [_vp, _vp, _f, _i, _i, _vp, _i, _vp, _vp, _vp]),
     "qh_sample_workspace_size": (_sz, [_i]),
     "qh_sample_top_p": (_i, [_vp, _i, _f, _f, _f, _vp, _i, _vp, _i, _i, _vp, _i, _u64, _vp, _vp,
                              _vp, _vp, _vp, _i, _vp, _vp]),

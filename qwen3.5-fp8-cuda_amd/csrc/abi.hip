@@ -682,6 +682,24 @@ QH_EXPORT int qh_lm_head_argmax(const void* x, const float* norm_w, float eps, i
   return check_launch("qh_lm_head_argmax");
 }
 
+// lm_head over M rows: xn = bf16 (1+w) RMSNorm of x's rows (x itself when norm_w
+// is null), logits[m] = bf16(xn[m] . w^T).
+QH_EXPORT int qh_lm_head_rows(const void* x, const float* norm_w, float eps, int M, int K, const void* w, int N,
+                              void* xn, void* logits, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (N <= 0 || !x || !w || !logits || (norm_w && !xn)) {
+    qh_set_error("qh_lm_head_rows: N=%d, or a null pointer", N);
+    return -1;
+  }
+  if (K <= 0 || K % 64 != 0) {
+    qh_set_error("qh_lm_head_rows: K=%d must be a positive multiple of 64", K);
+    return -1;
+  }
+  if (norm_w) qh_launch_rmsnorm_rows(x, norm_w, xn, M, K, eps, stream);
+  if (qh_launch_head_rows(norm_w ? xn : x, w, logits, M, N, K, stream) != 0) return -1;
+  return check_launch("qh_lm_head_rows");
+}
+
 QH_EXPORT size_t qh_sample_workspace_size(int V) { return qh_sample_workspace_bytes(V); }
 
 // Nucleus sampling of one bf16 logits row (main.py:49-87) on the device.

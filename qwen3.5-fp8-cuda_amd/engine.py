@@ -518,7 +518,12 @@ class Qwen35FP8Engine:
             # every kept position but the last: logits only (no token, position
             # or history side effects)
             out = torch.empty(keep, cfg.vocab_size, dtype=torch.bfloat16, device=self.device)
-            for j in range(keep - 1):
+            rows = H % 64 == 0 and self.w.lm_head.data_ptr() % 16 == 0
+            if rows:   # all of them in one pass over the head's weights (hn is free by now)
+                abi.check(L.qh_lm_head_rows(abi.ptr(h[M - keep]), abi.ptr(self.w.norm_f), eps, keep - 1, H,
+                                            abi.ptr(self.w.lm_head), cfg.vocab_size, abi.ptr(hn), abi.ptr(out),
+                                            st), "lm_head_rows")
+            for j in range(0 if rows else keep - 1):
                 r = M - keep + j
                 abi.check(L.qh_lm_head_argmax(
                     abi.ptr(h[r]), abi.ptr(self.w.norm_f), eps, H, abi.ptr(self.w.lm_head),

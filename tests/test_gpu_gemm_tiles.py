@@ -94,3 +94,27 @@ def test_gemm_tile_segments(M):
     abi.check(lib.qh_gemm_e4m3_grouped(abi.ptr(dx), M, K, 4, *args, 0, None, 0, abi.stream_handle()), "grouped")
     for (w, s), y, n in zip(segs, ys, ns):
         check(y, *product(x, w, s), K, f"{M} rows, {n} columns")
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 100, 64), (2, 1003, 256), (32, 260, 2560), (33, 1001, 192), (64, 4096, 256),
+                                   (65, 130, 320), (129, 1027, 2560), (300, 520, 128)])
+def test_lm_head_rows(M, N, K):
+    """Row blocks of 32, 64 and 128 by 128 columns with ragged ends; a row's logits are the same
+    bits however many rows come with it."""
+    g = gen(M + N + K)
+    x, w, nw = bf(randn(g, M, K)).to(DEV), bf(randn(g, N, K, std=0.02)).to(DEV), randn(g, K, std=0.02).to(DEV)
+    lib = abi.load()
+    xn, ref_xn = torch.empty(2, M, K, dtype=torch.bfloat16, device=DEV).unbind(0)
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+
+    def run(xx, yy, m):
+        abi.check(lib.qh_lm_head_rows(abi.ptr(xx), abi.ptr(nw), 1e-6, m, K, abi.ptr(w), N, abi.ptr(xn), abi.ptr(yy),
+                                      abi.stream_handle()), "lm_head_rows")
+    run(x, y, M)
+    abi.check(lib.qh_rmsnorm(abi.ptr(x), abi.ptr(nw), abi.ptr(ref_xn), M, K, 1e-6, abi.stream_handle()), "rmsnorm")
+    assert torch.equal(xn, ref_xn)
+    d, dw = xn.double(), w.double()
+    check(y, d @ dw.t(), d.abs() @ dw.abs().t(), K, "lm_head rows")
+    last = torch.empty(1, N, dtype=torch.bfloat16, device=DEV)
+    run(x[M - 1:].contiguous(), last, 1)
+    assert torch.equal(last[0], y[M - 1])
