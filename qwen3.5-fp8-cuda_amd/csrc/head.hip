@@ -11,13 +11,18 @@
 
 namespace {
 
-// Tiles of 32, 64 or 128 rows by 128 columns, four waves, two workgroups per
-// CU (LDS); one K group and the same order of K steps in each, so a row's
-// logits do not depend on how many rows there are.  Up to 128 rows the weight
-// stream bounds it, above that the matrix products.
+// One K group and the same order of K steps in every shape, so a row's logits
+// do not depend on how many rows there are.  Up to 128 rows the weight stream
+// bounds it (a plain read of it: 186 us), above that the matrix products.  us
+// at 248320 x 2560, the shapes by their row ranges:
+//   8 / 32 rows     32 x 128   218 / 233  (64 x 128: 220 / 233)
+//   64 rows         64 x 128   253        (128 x 128: 257)
+//   95 / 128 rows   128 x 256  264 / 275  (128 x 128: 280 / 299)
+//   512 rows        128 x 128  746        (128 x 256: 778; 256 x 128: 764)
 using Head32 = qh_tile::Cfg<2, 2, 1, 4, 1, 64, 3, 2>;
 using Head64 = qh_tile::Cfg<4, 2, 1, 4, 1, 64, 3, 2>;
-using Head128 = qh_tile::Cfg<4, 4, 2, 2, 1, 64, 2, 2>;
+using Head128 = qh_tile::Cfg<4, 4, 2, 4, 1, 64, 3, 2>;
+using HeadMany = qh_tile::Cfg<4, 4, 2, 2, 1, 64, 2, 2>;
 
 // Workgroup b runs on XCD b % 8, which takes the x-th eighth of the tiles, row
 // tile fastest: the row tiles of a column run together and share its weights.
@@ -71,6 +76,7 @@ int qh_launch_head_rows(const void* x, const void* w, void* logits, int M, int N
   const uint16_t *xa = (const uint16_t*)x, *wa = (const uint16_t*)w;
   if (M <= 32) launch<Head32>(xa, wa, (uint16_t*)logits, M, N, K, st);
   else if (M <= 64) launch<Head64>(xa, wa, (uint16_t*)logits, M, N, K, st);
-  else launch<Head128>(xa, wa, (uint16_t*)logits, M, N, K, st);
+  else if (M <= 128) launch<Head128>(xa, wa, (uint16_t*)logits, M, N, K, st);
+  else launch<HeadMany>(xa, wa, (uint16_t*)logits, M, N, K, st);
   return 0;
 }
