@@ -606,6 +606,121 @@ __global__ __launch_bounds__(256) void gdn_norm_gates_kernel(QhGdnPrepParams p) 
   }
 }
 
+// ---- conv, l2norm and gates in one pass -------------------------------------
+// One thread per 8 channels (16-byte accesses) and T consecutive tokens, whose
+// inputs slide through registers: T + 3 loads for T outputs where a thread per
+// token takes 4 T.  16 lanes hold the 128 channels of a head, so a q or k
+// head's sum of squares is a 16-lane DPP sum and its normalised row is stored
+// from the same registers.  Blocks of 4 waves, 16 T tokens; blockIdx.y < C / 128:
+// that row of 128 channels, C / 128: the gates.  The conv ring (window positions
+// before the prompt) is read by the threads of token 0's wave only, and they
+// store its new contents after their own outputs, which depend on their reads.
+// Bound by the SiLU's arithmetic from a few hundred tokens (3700 tokens: 47 us,
+// 60 + 34 as a conv and a norm kernel with expf and IEEE divisions; the bytes
+// alone 35), by one round trip below (128 tokens: 4.9 us, 5.4 + 3.8).
+template <int T>
+__global__ __launch_bounds__(256) void gdn_front_kernel(QhGdnPrepParams p) {
+  const int wv = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int rows = p.C >> 7;
+  if ((int)blockIdx.y == rows) {  // gates of the block's 16 T tokens
+    const int m0 = (int)blockIdx.x * 16 * T, n = min(16 * T, p.M - m0) * p.Hv;
+    for (int i = threadIdx.x; i < n; i += 256) {
+      const int h = i % p.Hv;
+      const size_t at = (size_t)m0 * p.Hv + i;
+      const float a = bf2f(p.a[at]), b = bf2f(p.b[at]);
+      p.g[at] = -expf(p.A_log[h]) * qh_softplus(a + p.dt_bias[h]);
+      p.beta[at] = f2bf(qh_sigmoid(b));
+    }
+    return;
+  }
+  const int m0 = (wv * 4 + (lane >> 4)) * T, c0 = (int)blockIdx.y * 128 + (lane & 15) * 8;
+  if (m0 >= p.M) return;  // uniform over the 16 lanes of a token group
+  const u32x4* wq = (const u32x4*)(p.conv_w + (size_t)c0 * 4);
+  u32x4* ring = (u32x4*)(p.conv_ring + (size_t)c0 * 4);
+  const u32x4 wv4[4] = {wq[0], wq[1], wq[2], wq[3]};
+  u32x4 x[T + 3];  // x[j]: token m0 - 3 + j
+#pragma unroll
+  for (int j = 0; j < T + 3; ++j) {
+    const int t = min(max(m0 - 3 + j, 0), p.M - 1);
+    x[j] = *(const u32x4*)(p.mixed + (size_t)t * p.C + c0);
+  }
+  u32x4 old[4] = {}, last[4] = {};
+  if (m0 < 3) {  // window positions before the prompt: slot (past + t) % 4 of each channel
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      old[q] = ring[q];
+      last[q] = *(const u32x4*)(p.mixed + (size_t)max(p.M - 1 - q, 0) * p.C + c0);
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int t = m0 - 3 + j;
+      if (t < 0) {
+        const int s = (p.past + t) & 3, sh = 16 * (s & 1);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {  // old[q]: channel 2 q in words x, y and 2 q + 1 in z, w, two slots a word
+          const uint32_t e0 = s < 2 ? old[q].x : old[q].y, e1 = s < 2 ? old[q].z : old[q].w;
+          x[j][q] = ((e0 >> sh) & 0xFFFFu) | ((e1 >> sh) << 16);
+        }
+      }
+    }
+  }
+  const bool is_qk = (int)blockIdx.y < 2 * p.Hk;
+  uint16_t* ndst = (int)blockIdx.y < p.Hk ? p.qn : p.kn;
+  const int kh = (int)blockIdx.y % p.Hk;
+#pragma unroll
+  for (int k = 0; k < T; ++k) {
+    const int m = m0 + k;
+    u32x4 out;
+    float ss = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float r2[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int e = 4 * (2 * q + h);  // tap j of channel 2 q + h is element e + j of the 32
+        auto wt = [&](int j) {
+          const uint32_t word = wv4[(e + j) >> 3][((e + j) >> 1) & 3];
+          return (j & 1) ? bf_hi(word) : bf_lo(word);
+        };
+        auto xv = [&](int d) { return h ? bf_hi(x[k + 3 - d][q]) : bf_lo(x[k + 3 - d][q]); };
+        float acc = wt(3) * xv(0);
+        acc = fmaf(wt(2), xv(1), acc);
+        acc = fmaf(wt(1), xv(2), acc);
+        acc = fmaf(wt(0), xv(3), acc);
+        r2[h] = qh_silu_bf(rbf(acc));
+      }
+      out[q] = pack_bf2(r2[0], r2[1]);
+      const float y0 = bf_lo(out[q]), y1 = bf_hi(out[q]);
+      ss += rbf(y0 * y0) + rbf(y1 * y1);
+    }
+    if (m < p.M) *(u32x4*)(p.y + (size_t)m * p.C + c0) = out;
+    if (is_qk) {
+      ss = column_sum<16>(ss);
+      const float inv = rbf(rsqrtf(rbf(rbf(ss) + 1e-6f)));
+      u32x4 nv;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) nv[q] = pack_bf2(bf_lo(out[q]) * inv, bf_hi(out[q]) * inv);
+      if (m < p.M) *(u32x4*)(ndst + ((size_t)m * p.Hk + kh) * 128 + (lane & 15) * 8) = nv;
+    }
+  }
+  if (m0 == 0) {  // the ring's last four positions (older slots of a short prompt stay)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const int t = p.M - 1 - d, s = (p.past + t) & 3, sh = 16 * (s & 1);
+      const uint32_t m_lo = t >= 0 && s < 2 ? 0xFFFFu << sh : 0u, m_hi = t >= 0 && s >= 2 ? 0xFFFFu << sh : 0u;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t c_lo = last[d][q] & 0xFFFFu, c_hi = last[d][q] >> 16;
+        const uint32_t v0 = c_lo | (c_lo << 16), v1 = c_hi | (c_hi << 16);
+        old[q] = u32x4{(old[q].x & ~m_lo) | (v0 & m_lo), (old[q].y & ~m_hi) | (v0 & m_hi),
+                       (old[q].z & ~m_lo) | (v1 & m_lo), (old[q].w & ~m_hi) | (v1 & m_hi)};
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ring[q] = old[q];
+  }
+}
+
 // ---- recurrent scan: one wave per (head, COLS value columns) ---------------
 // Lane l owns value column j = 8 cg + (l >> 3) of head h and state rows
 // 16 (l & 7) .. +16 of it, so the two sums over the key dimension (S^T k and
@@ -707,21 +822,28 @@ __global__ __launch_bounds__(64) void gdn_scan_kernel(QhGdnScanParams p) {
   for (int i = 0; i < RPT; ++i) col[(size_t)(r * RPT + i) * DV] = S[i];
 }
 
-// ---- gated RMSNorm of the scan output, in place: one 128-thread block per
-// (token, head) (main.py:1152-1158) --------------------------------------------
-// One wave per (token, head), four per block, no LDS or barrier: lane j
-// holds elements j and j + 64 and the two 64-element sums are added as the
-// two-wave kernel below does, so the results are the same bit for bit.
+// ---- gated RMSNorm of the scan output, in place (main.py:1152-1158) -------------
+// 16 lanes per (token, head), 8 elements each in 16-byte accesses (a wave per
+// row in 2-byte ones took 27 us at 3700 tokens; the bytes alone 18).
 __global__ __launch_bounds__(256) void gdn_gated_norm_wave_kernel(QhGdnScanParams p) {
-  const int idx = (int)blockIdx.x * 4 + (threadIdx.x >> 6), j = threadIdx.x & 63;
-  if (idx >= p.M * p.Hv) return;
+  const long idx = (long)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const int j = (threadIdx.x & 15) * 8;
+  if (idx >= (long)p.M * p.Hv) return;
   const size_t o = (size_t)idx * 128 + j;  // token idx / Hv, head idx % Hv: rows of Hv * 128
-  const float c0 = bf2f(p.out[o]), c1 = bf2f(p.out[o + 64]);
-  const float z0 = bf2f(p.z[o]), z1 = bf2f(p.z[o + 64]);
-  const float w0 = bf2f(p.norm_w[j]), w1 = bf2f(p.norm_w[j + 64]);
-  const float rs = rsqrtf((wave_sum(c0 * c0) + wave_sum(c1 * c1)) / 128.0f + p.eps);
-  p.out[o] = f2bf(rbf(rbf(c0 * rs) * w0) * rbf(qh_silu(z0)));
-  p.out[o + 64] = f2bf(rbf(rbf(c1 * rs) * w1) * rbf(qh_silu(z1)));
+  const u32x4 cv = *(const u32x4*)(p.out + o), zv = *(const u32x4*)(p.z + o), wv = *(const u32x4*)(p.norm_w + j);
+  float ss = 0.0f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    ss = fmaf(bf_lo(cv[q]), bf_lo(cv[q]), ss);
+    ss = fmaf(bf_hi(cv[q]), bf_hi(cv[q]), ss);
+  }
+  const float rs = rsqrtf(column_sum<16>(ss) / 128.0f + p.eps);
+  u32x4 y;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    y[q] = pack_bf2(rbf(rbf(bf_lo(cv[q]) * rs) * bf_lo(wv[q])) * rbf(qh_silu_bf(bf_lo(zv[q]))),
+                    rbf(rbf(bf_hi(cv[q]) * rs) * bf_hi(wv[q])) * rbf(qh_silu_bf(bf_hi(zv[q]))));
+  *(u32x4*)(p.out + o) = y;
 }
 __global__ __launch_bounds__(128) void gdn_gated_norm_kernel(QhGdnScanParams p) {
   __shared__ float red2[2];
@@ -735,56 +857,6 @@ __global__ __launch_bounds__(128) void gdn_gated_norm_kernel(QhGdnScanParams p) 
   const float rs = rsqrtf((red2[0] + red2[1]) / 128.0f + p.eps);
   const float normed = rbf(rbf(core * rs) * nw);
   p.out[o] = f2bf(normed * rbf(qh_silu(zv)));
-}
-
-// 8 channels per thread (16-byte loads and store; C % 8 == 0 and aligned
-// rows), the same arithmetic per channel as gdn_conv_kernel.
-__global__ __launch_bounds__(256) void gdn_conv8_kernel(QhGdnPrepParams p) {
-  const int C8 = p.C >> 3;
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (size_t)p.M * C8) return;
-  const int m = (int)(i / (size_t)C8), c0 = (int)(i - (size_t)m * C8) * 8;
-  // taps of channels c0 .. c0 + 7: w[c * 4 + j], 64 contiguous bytes
-  const u32x4* wq = (const u32x4*)(p.conv_w + (size_t)c0 * 4);
-  const u32x4 wv[4] = {wq[0], wq[1], wq[2], wq[3]};
-  float x[4][8];  // x[d][k]: token m - d, channel c0 + k
-#pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    const int t = m - d;
-    if (t >= 0) {
-      const u32x4 v = *(const u32x4*)(p.mixed + (size_t)t * p.C + c0);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        x[d][2 * q] = bf_lo(v[q]);
-        x[d][2 * q + 1] = bf_hi(v[q]);
-      }
-    } else {
-#pragma unroll
-      for (int k = 0; k < 8; ++k) x[d][k] = bf2f(p.conv_ring[(size_t)(c0 + k) * 4 + ((p.past + t) & 3)]);
-    }
-  }
-  u32x4 out;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    float r2[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int k = 2 * q + h;
-      // w of channel k, tap j: word (4 k + j) / 2 of the 16 words
-      auto wt = [&](int j) {
-        const int e = 4 * k + j;
-        const uint32_t word = wv[e >> 3][(e >> 1) & 3];
-        return (e & 1) ? bf_hi(word) : bf_lo(word);
-      };
-      float acc = wt(3) * x[0][k];
-      acc = fmaf(wt(2), x[1][k], acc);
-      acc = fmaf(wt(1), x[2][k], acc);
-      acc = fmaf(wt(0), x[3][k], acc);
-      r2[h] = qh_silu(rbf(acc));
-    }
-    out[q] = (uint32_t)f2bf(r2[0]) | ((uint32_t)f2bf(r2[1]) << 16);
-  }
-  *(u32x4*)(p.y + (size_t)m * p.C + c0) = out;
 }
 
 // 8 elements per thread (16-byte loads and store), same arithmetic.
@@ -869,17 +941,21 @@ int qh_launch_gdn_prep(const QhGdnPrepParams& p, hipStream_t st) {
     return -1;
   }
   if (p.M <= 0) return 0;
-  const size_t n = (size_t)p.M * p.C;
-  // 8 channels per thread from 512 tokens (3700 tokens: 72.8 -> 49.6 us);
-  // below that the thread-per-channel kernel's parallelism wins (128 tokens:
-  // 4.8 against 6.1 us)
-  if (p.M >= 512 && p.C % 8 == 0 && (uintptr_t)p.mixed % 16 == 0 && (uintptr_t)p.y % 16 == 0 &&
-      (uintptr_t)p.conv_w % 16 == 0) {
-    const size_t n8 = n / 8;
-    hipLaunchKernelGGL(gdn_conv8_kernel, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, st, p);
-  } else {
-    hipLaunchKernelGGL(gdn_conv_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p);
+  // One pass when every row can be moved in 16-byte pieces: 8 tokens per thread
+  // from 512 tokens, 1 below (the threads of a short prompt are its
+  // parallelism).
+  const void* al[] = {p.mixed, p.y, p.conv_w, p.conv_ring, p.qn, p.kn};
+  bool aligned = true;
+  for (const void* q : al) aligned = aligned && (uintptr_t)q % 16 == 0;
+  if (aligned) {
+    const int T = p.M >= 512 ? 8 : 1;
+    const dim3 grid((unsigned)((p.M + 16 * T - 1) / (16 * T)), (unsigned)(p.C / 128 + 1));
+    if (T == 8) hipLaunchKernelGGL(gdn_front_kernel<8>, grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL(gdn_front_kernel<1>, grid, dim3(256), 0, st, p);
+    return 0;
   }
+  const size_t n = (size_t)p.M * p.C;
+  hipLaunchKernelGGL(gdn_conv_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p);
   hipLaunchKernelGGL(gdn_norm_gates_kernel, dim3((unsigned)(((long)p.M * (2 * p.Hk + 1) + 3) / 4)), dim3(256), 0, st,
                      p);
   return 0;
@@ -899,9 +975,9 @@ int qh_launch_gdn_scan(const QhGdnScanParams& p, hipStream_t st) {
 
 int qh_launch_gdn_gated_norm(const QhGdnScanParams& p, hipStream_t st) {
   if (p.M <= 0) return 0;
-  if (p.dv == 128) {
+  if (p.dv == 128 && (uintptr_t)p.out % 16 == 0 && (uintptr_t)p.z % 16 == 0 && (uintptr_t)p.norm_w % 16 == 0) {
     const long n = (long)p.M * p.Hv;
-    hipLaunchKernelGGL(gdn_gated_norm_wave_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, p);
+    hipLaunchKernelGGL(gdn_gated_norm_wave_kernel, dim3((unsigned)((n + 15) / 16)), dim3(256), 0, st, p);
   } else {
     hipLaunchKernelGGL(gdn_gated_norm_kernel, dim3(p.M, p.Hv), dim3(128), 0, st, p);
   }

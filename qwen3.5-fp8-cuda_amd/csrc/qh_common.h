@@ -209,6 +209,24 @@ __device__ __forceinline__ void reset_counter(unsigned* counter) {
 // flips and a per-step bias against the reference's fp32 torch ops.
 __device__ __forceinline__ float qh_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float qh_silu(float x) { return x / (1.0f + expf(-x)); }
+// SiLU whose argument is a bf16 value and whose result is rounded to bf16, for
+// loops that its arithmetic bounds: e^-x as 2^t with the rounding of
+// t = -x log2(e) corrected to first order, and one Newton step on the hardware
+// reciprocal's quotient, 12 instructions in place of expf's and the IEEE
+// division's 25.  Over all finite bf16 arguments it rounds to the bf16 value
+// that 64-bit arithmetic gives at least as often as fp32 arithmetic with expf
+// does (test_conv_silu_every_argument).  Above 88 it is x (as in fp32, infinity
+// included), below -88 zero or a denormal; NaN stays NaN.
+__device__ __forceinline__ float qh_silu_bf(float x) {
+  const float a = fminf(-x, 88.0f);
+  const float t = a * 1.44269502f;                                // log2(e), high part
+  const float c = fmaf(a, 1.92596299e-8f, fmaf(a, 1.44269502f, -t));  // low part and t's rounding
+  const float e = __builtin_amdgcn_exp2f(t);
+  const float d = 1.0f + fmaf(e, c * 0.693147182f, e);
+  const float q = x * __builtin_amdgcn_rcpf(d);
+  const float y = fmaf(fmaf(-q, d, x), __builtin_amdgcn_rcpf(d), q);
+  return x > 88.0f ? x : y;
+}
 // SiLU on the fast exponential, for per-element loops on a kernel's critical
 // path (the gated RMSNorm prologue of the decode output projection).
 // The reciprocal is the hardware v_rcp_f32 (about 1 ulp) in place of the IEEE
