@@ -16,6 +16,7 @@
 #include "qh_prefill.h"
 
 #include <algorithm>
+#include <utility>
 
 namespace {
 
@@ -251,55 +252,58 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(QhAttnPrefillParams p
 // 4 kvh + w of the GQA group, so the 4 waves share every K / V tile in LDS.
 // Tiles of 64 key positions; rows at or past the workgroup's last key (and
 // past the prompt) read as zeros through the range-checked buffer resources.
-// The next tile's K / V rows are loaded into registers while the current tile
-// is computed.
 //
 // Scores are computed transposed, S^T = K Q^T on v_mfma_f32_32x32x16_bf16 (A = K
 // rows, B = Q^T), so each lane owns one query row (lane % 32) and 16 of a
 // 32-position block's scores: the row max and sum need one exchange with the
 // partner lane (lane ^ 32, v_permlane32_swap).  The output is also transposed,
-// O^T = V^T P^T (A = the V tile stored transposed in LDS, B = P^T), so a
-// lane's 128 accumulators are its own query row and the online-softmax
-// rescale stays in the lane.
+// O^T = V^T P^T (A = the V tile, transposed as it is read by
+// ds_read_b64_tr_b16, B = P^T), so a lane's 128 accumulators are its own query
+// row and the online-softmax rescale stays in the lane.
+//
+// What bounds it: 104 matrix products of 32 cycles per tile and wave.  The
+// accumulators leave room for one wave per SIMD, so that nothing but the
+// wave's own instructions can fill the matrix unit's time: each product is
+// followed by a slice of vector work that does not depend on it (the softmax
+// of tile t beside the scores of tile t + 1, that tile's mask and row max
+// beside the output of tile t).  K and V come by direct-to-LDS loads into two
+// stages each, requested two tiles ahead for K and V of the tile before.
+// Two thirds of a tile's 4.9 k cycles are products (a lone wave issues one
+// instruction per 5 cycles, and about 5 of them ride under a product); with
+// every step in turn and register-staged tiles it took 10 k.  3700 tokens: 265
+// -> 182 us, 512 tokens after 3072 228 -> 131 us, 256 tokens 35.5 -> 25 us, of
+// which 18 us are a workgroup's start (query load and split) and end.
 //
 // The rescale is lazy: the exponentials use a per-row reference max that is
 // raised only when some row's running max passes it by more than kFaSlack, so
 // p <= e^kFaSlack and O / l is unchanged up to fp32 rounding; most tiles skip
-// the 128-accumulator rescale.  Only tiles that reach past the workgroup's
-// first query position apply the causal mask.
+// the 128-accumulator rescale.
 //
 // Precision as the reference's fp32 q . k, softmax and P . v: q (fp32) and P
 // (fp32) enter as hi + lo bf16 pairs (hi = bf16(x), lo = bf16(x - hi), about
 // 16 mantissa bits), each pair two matrix-core products that are exact in
 // fp32; k and v are bf16 already.  q is scaled by 1/16 = 256^-1/2 first
-// (exact).  The q hi parts stay in registers, the lo parts in a per-wave LDS
-// area; a 16-dimension block's lo term is computed only when it is nonzero for
-// some lane of the wave (the head-norm output is a bf16 value in every
-// dimension RoPE does not rotate).
-constexpr int kFaTile = 64;                    // key positions per tile
-constexpr int kFaKRow = 256 * 2 + 16;          // padded K row in LDS (bytes)
-constexpr int kFaVRow = kFaTile * 2 + 16;      // padded V^T row in LDS (bytes)
-constexpr int kFaQRow = 256 * 2 + 16;          // padded q lo row in LDS (bytes)
-constexpr int kFaV0 = kFaTile * kFaKRow;                       // 33,792
-constexpr int kFaQ0 = kFaV0 + 256 * kFaVRow;                   // 70,656
-constexpr int kFaLds = kFaQ0 + 4 * 32 * kFaQRow;               // 138,240 B
+// (exact).  q stays in registers; the head-norm output is a bf16 value in
+// every dimension RoPE does not rotate, so with lo parts in the first 64
+// dimensions only (RoPE's) the other 12 blocks' lo products are left out.
+//
+// LDS rows are 512 bytes unpadded, in 16-byte slots swizzled by row: K chunk c
+// of row r in slot c ^ (r % 16) (a read takes one chunk of 32 rows), V in slot
+// c ^ 4 (r % 4) (a transposing read takes 64 bytes of 4 rows).
+constexpr int kFaTile = 64;                         // key positions per tile
+constexpr int kFaStage = kFaTile * 512;             // one K or V tile
+constexpr int kFaV0 = 2 * kFaStage;                 // K stages, then V stages
+constexpr int kFaLds = 4 * kFaStage;                // 131,072 B
 constexpr float kFaSlack = 8.0f;
+constexpr float kFaLog2e = 1.44269504f;
 
 typedef float v16f_fa __attribute__((ext_vector_type(16)));
 typedef __bf16 v8bf_fa __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) void* fa_lds_ptr;
 
-__device__ __forceinline__ uint32_t pack_bf2(float a, float b) {
-  return (uint32_t)f2bf(a) | ((uint32_t)f2bf(b) << 16);
-}
-// 8 fp32 -> hi (bf16 of each) and lo (bf16 of each residual), packed
-__device__ __forceinline__ void split8(const float (&v)[8], u32x4& hi, u32x4& lo) {
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float a = v[2 * q], b = v[2 * q + 1];
-    const float ah = rbf(a), bh = rbf(b);
-    hi[q] = (__float_as_uint(ah) >> 16) | (__float_as_uint(bh) & 0xFFFF0000u);
-    lo[q] = pack_bf2(a - ah, b - bh);
-  }
+// (one v_cvt_pk_bf16_f32)
+__device__ __forceinline__ uint32_t pack_pair(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(qh_f32x2{a, b}, qh_bf16x2));
 }
 // both lanes of a (lane, lane ^ 32) pair get max / sum of their two values
 __device__ __forceinline__ float pair_max(float x) {
@@ -310,235 +314,452 @@ __device__ __forceinline__ float pair_sum(float x) {
   const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
+// LDS reads the compiler does not count against the direct-to-LDS loads in
+// flight; every one is waited for by count before its first use.
+template <int OFF>
+__device__ __forceinline__ u32x4 fa_read(uint32_t a) {
+  u32x4 v;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(a), "n"(OFF) : "memory");
+  return v;
+}
+// 16 lanes' 8-byte reads (lane i: row i / 4, columns 4 (i % 4) .. + 3 of a 4 x 16
+// block) transposed: lane i gets column i, rows 0 .. 3
+template <int OFF>
+__device__ __forceinline__ u32x2 fa_read_tr(uint32_t a) {
+  u32x2 v;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(a), "n"(OFF) : "memory");
+  return v;
+}
+template <int N>
+__device__ __forceinline__ void fa_lds_wait() {
+  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
+}
+template <typename T>
+__device__ __forceinline__ void fa_settle(T& v) { asm volatile("" : "+v"(v)); }
 
-__global__ __launch_bounds__(256) void attn_prefill_mfma_kernel(QhAttnPrefillParams p) {
-  extern __shared__ __align__(16) uint8_t smem[];
-  uint8_t* sK = smem;
-  uint8_t* sV = smem + kFaV0;
+template <int... I, typename F>
+__device__ __forceinline__ void fa_unroll(std::integer_sequence<int, I...>, F f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void fa_for(F f) { fa_unroll(std::make_integer_sequence<int, N>{}, f); }
+
+// What a wave holds through the tile loop.
+template <int NL>
+struct FaWave {
+  v16f_fa o[8];               // O^T: dims 32 d .. + 31, the lane's query
+  u32x4 qhi[16], qlo[NL];     // Q^T operands of 16-dimension blocks
+  v16f_fa c0, c1;             // scores of the tile whose softmax is next, masked
+  v16f_fa n0, n1;             // scores of the tile after it
+  u32x4 ka[4][2];             // K operands, four blocks in flight
+  u32x2 va[2][8][2];          // V operands of two 16-position steps
+  u32x4 phi[4], plo[4];       // P^T operands
+  float rest[4][2];           // p - bf16(p) of the operand block being split
+  uint32_t kaddr[8], vaddr[4];
+  float mref, mlog, lsum, tmax;  // mlog: mref log2(e)
+  int lim;                    // last unmasked position, less the 4 h of the lane's scores
+};
+
+// K operands of 16-dimension block KK (both 32-position halves)
+template <int NL, int KK>
+__device__ __forceinline__ void fa_k_read(FaWave<NL>& w) {
+  w.ka[KK % 4][0] = fa_read<(KK / 8) * 256>(w.kaddr[KK % 8]);
+  w.ka[KK % 4][1] = fa_read<(KK / 8) * 256 + 32 * 512>(w.kaddr[KK % 8]);
+}
+// read I (of 16) of the V operands of 16-position step KK
+template <int NL, int KK, int I>
+__device__ __forceinline__ void fa_v_read(FaWave<NL>& w) {
+  constexpr int d = I / 2, j = I % 2;
+  w.va[KK % 2][d][j] = fa_read_tr<(16 * KK + 8 * j) * 512 + (d / 4) * 256>(w.vaddr[d % 4]);
+}
+
+// Stage ST of softmax piece ID (0 .. 47) of the tile in c0, c1: operand block
+// ID / 12's eight exponentials and four splits.  A lane's scores b .. b + 7 are
+// the positions 4 h + 0 .. 3 and 8 + 4 h + 0 .. 3 of 16; they enter the products in
+// that order, and the V reads follow it.
+template <int NL, int ID, int ST>
+__device__ __forceinline__ void fa_piece(FaWave<NL>& w) {
+  if constexpr (ID >= 0 && ID < 48) {
+    constexpr int j = ID / 12, q = ID % 12, b = 8 * (j & 1);
+    v16f_fa& s = j < 2 ? w.c0 : w.c1;
+    if constexpr (q < 8) {
+      if constexpr (ST == 0) s[b + q] = fmaf(s[b + q], kFaLog2e, -w.mlog);
+      if constexpr (ST == 1) s[b + q] = __builtin_amdgcn_exp2f(s[b + q]);
+      if constexpr (ST == 2) w.lsum += s[b + q];
+    } else {
+      constexpr int i = q - 8;
+      const float x = s[b + 2 * i], y = s[b + 2 * i + 1];
+      if constexpr (ST == 0) w.phi[j][i] = pack_pair(x, y);
+      if constexpr (ST == 1) {
+        w.rest[i][0] = bf_lo(w.phi[j][i]);
+        w.rest[i][1] = bf_hi(w.phi[j][i]);
+      }
+      if constexpr (ST == 2) {
+        w.rest[i][0] = x - w.rest[i][0];
+        w.rest[i][1] = y - w.rest[i][1];
+      }
+      if constexpr (ST == 3) w.plo[j][i] = pack_pair(w.rest[i][0], w.rest[i][1]);
+    }
+  }
+}
+// Softmax step T (0 .. 50): four pieces' stages that do not depend on each other
+// (a lone wave waits out every dependent pair).
+template <int NL, int T>
+__device__ __forceinline__ void fa_softmax(FaWave<NL>& w) {
+  fa_piece<NL, T, 0>(w);
+  fa_piece<NL, T - 1, 1>(w);
+  fa_piece<NL, T - 2, 2>(w);
+  fa_piece<NL, T - 3, 3>(w);
+}
+__device__ __forceinline__ float fa_max3(float a, float b, float c) {
+  float d;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+  return d;
+}
+// Takes scores E of both halves of the next tile over into vector registers,
+// with their row max.  (By asm: the compiler would leave them in accumulation
+// registers and move them back and forth around the mask.  It sees no hazard
+// here, so the caller keeps the products that wrote them at least 16 products,
+// or 64 idle cycles, away.)
+template <int NL, int E>
+__device__ __forceinline__ void fa_take(FaWave<NL>& w) {
+  float x, y;
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(w.n0[E]));
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(y) : "a"(w.n1[E]));
+  w.c0[E] = x;
+  w.c1[E] = y;
+  w.tmax = E == 0 ? fmaxf(w.c0[E], w.c1[E]) : fa_max3(w.tmax, w.c0[E], w.c1[E]);
+}
+// Causal mask (positions past lim) of the tile in c0, c1, with the row max of what is left.  Score
+// e of half nt is position 32 nt + 8 (e / 4) + 4 h + e % 4 of the tile.
+template <int NL>
+__device__ __forceinline__ void fa_mask(FaWave<NL>& w, int lim) {
+  w.tmax = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const int idx = 8 * (e >> 2) + (e & 3);
+    w.c0[e] = idx <= lim ? w.c0[e] : -INFINITY;
+    w.c1[e] = idx + 32 <= lim ? w.c1[e] : -INFINITY;
+    w.tmax = fa_max3(w.tmax, w.c0[e], w.c1[e]);
+  }
+}
+
+constexpr int fa_v_step(int kk) { return kk >= 5 && kk < 13; }
+
+// S^T of the tile at kaddr into n0, n1; with SOFT, the first 38 steps of the
+// current tile's softmax and V operands' first reads between the products.
+// The reads of blocks 0 .. 2 are in flight.
+template <int NL, bool SOFT>
+__device__ __forceinline__ void fa_scores(FaWave<NL>& w) {
+  constexpr int NP = 32 + 2 * NL;  // products
+  fa_for<16>([&](auto kc) {
+    constexpr int kk = decltype(kc)::value;
+    // K reads of block kk + 3 go out in block kk, V reads of step 0 in blocks
+    // 5 .. 12, two each: waited for are all reads older than block kk's youngest
+    constexpr int k_after = (kk < 14 ? 2 : 15 - kk) * 2;
+    constexpr int v_after = SOFT ? 2 * (fa_v_step(kk - 3) + fa_v_step(kk - 2) + fa_v_step(kk - 1)) : 0;
+    fa_lds_wait<k_after + v_after>();
+    fa_settle(w.ka[kk % 4][0]);
+    fa_settle(w.ka[kk % 4][1]);
+    // the query operands live in accumulation registers: the vector ones are full
+    asm volatile("" : "+a"(w.qhi[kk]));
+    if constexpr (kk < NL && NL == 4) asm volatile("" : "+a"(w.qlo[kk]));
+    if constexpr (kk + 3 < 16) fa_k_read<NL, kk + 3>(w);
+    if constexpr (SOFT && fa_v_step(kk)) {
+      fa_v_read<NL, 0, 2 * (kk - 5)>(w);
+      fa_v_read<NL, 0, 2 * (kk - 5) + 1>(w);
+    }
+    constexpr int np = kk < NL ? 4 : 2, p0 = kk < NL ? 4 * kk : 4 * NL + 2 * (kk - NL);
+    fa_for<np>([&](auto ic) {
+      constexpr int i = decltype(ic)::value, at = p0 + i;
+      const v8bf_fa a = __builtin_bit_cast(v8bf_fa, w.ka[kk % 4][i & 1]);
+      v8bf_fa b;
+      if constexpr (i < 2) b = __builtin_bit_cast(v8bf_fa, w.qhi[kk]);
+      else b = __builtin_bit_cast(v8bf_fa, w.qlo[kk < NL ? kk : 0]);
+      v16f_fa& n = i & 1 ? w.n1 : w.n0;
+      if constexpr (kk == 0 && i < 2) n = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, v16f_fa{}, 0, 0, 0);
+      else n = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, n, 0, 0, 0);
+      if constexpr (SOFT) {
+        constexpr int t0 = 38 * at / NP, t1 = 38 * (at + 1) / NP;
+        fa_for<t1 - t0>([&](auto t) { fa_softmax<NL, t0 + decltype(t)::value>(w); });
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  });
+}
+
+// All nt tiles of the workgroup, the t-th of them at positions 64 at(t) on; those
+// from 64 tmask on need the causal mask.  On entry the first two K tiles and
+// then V tiles are requested; issue_k(t) and issue_v(t) request the t-th into
+// stage t % 2 (8 loads each).
+template <int NL, typename AT, typename IK, typename IV>
+__device__ __forceinline__ void fa_tiles(FaWave<NL>& w, int nt, int tmask, AT at, IK issue_k, IV issue_v) {
+#pragma unroll
+  for (int d = 0; d < 8; ++d)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) w.o[d][e] = 0.0f;
+  w.mref = w.mlog = -INFINITY;
+  w.lsum = 0.0f;
+  asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+  __builtin_amdgcn_s_barrier();  // K tiles 0 and 1 are in LDS
+  fa_k_read<NL, 0>(w);
+  fa_k_read<NL, 1>(w);
+  fa_k_read<NL, 2>(w);
+  fa_scores<NL, false>(w);
+  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  __builtin_amdgcn_s_barrier();  // V tile 0 is in LDS, K stage 0 is free
+  issue_k(2);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w.kaddr[i] ^= kFaStage;
+  fa_k_read<NL, 0>(w);
+  fa_k_read<NL, 1>(w);
+  fa_k_read<NL, 2>(w);
+  asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15\n\ts_nop 15");
+  fa_for<16>([&](auto e) { fa_take<NL, decltype(e)::value>(w); });
+  w.tmax = pair_max(w.tmax);
+  uint64_t raise = ~0ull;  // rows whose maximum passes the reference by more than the slack
+  for (int t = 0; t < nt; ++t) {
+    // tiles that reach past the workgroup's first query position
+    if (at(t) >= tmask) {
+      fa_mask(w, w.lim - kFaTile * at(t));
+      w.tmax = pair_max(w.tmax);
+      raise = __builtin_amdgcn_ballot_w64(w.tmax > w.mref + kFaSlack);
+    }
+    if (raise != 0) {
+      // every row's first tile has its first position unmasked, so mnew is finite
+      const float mnew = fmaxf(w.mref, w.tmax);
+      const float corr = mnew == w.mref ? 1.0f : __expf(w.mref - mnew);
+      w.lsum *= corr;
+      if (t > 0) {  // (O is zero before the first tile)
+#pragma unroll
+        for (int d = 0; d < 8; ++d)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            float x = w.o[d][e], tmp;
+            asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32_e32 %1, %2, %1\n\tv_accvgpr_write_b32 %0, %1"
+                         : "+a"(x), "=&v"(tmp)
+                         : "v"(corr));
+            w.o[d][e] = x;
+          }
+      }
+      w.mref = mnew;
+      w.mlog = mnew * kFaLog2e;
+    }
+    fa_scores<NL, true>(w);
+    // O^T += V^T P^T over 8 blocks of 32 dimensions; consecutive products go
+    // to different accumulators
+    fa_for<4>([&](auto kc) {
+      constexpr int kk = decltype(kc)::value;
+      fa_lds_wait<0>();
+#pragma unroll
+      for (int d = 0; d < 8; ++d) {
+        fa_settle(w.va[kk % 2][d][0]);
+        fa_settle(w.va[kk % 2][d][1]);
+      }
+      if constexpr (kk == 3) {
+        // the workgroup is done with K tile t + 1 and V tile t, and has K tile
+        // t + 2 and V tile t + 1
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        issue_k(t + 3);
+        issue_v(t + 2);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w.kaddr[i] ^= kFaStage;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w.vaddr[i] ^= kFaStage;
+      }
+      fa_for<16>([&](auto ic) {
+        constexpr int i = decltype(ic)::value, d = i % 8;
+        const u32x4 a = {w.va[kk % 2][d][0].x, w.va[kk % 2][d][0].y, w.va[kk % 2][d][1].x, w.va[kk % 2][d][1].y};
+        const u32x4 b = i < 8 ? w.phi[kk] : w.plo[kk];
+        w.o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_fa, a), __builtin_bit_cast(v8bf_fa, b),
+                                                         w.o[d], 0, 0, 0);
+        if constexpr (kk < 3 && i < 8) {
+          fa_v_read<NL, kk + 1, 2 * i>(w);
+          fa_v_read<NL, kk + 1, 2 * i + 1>(w);
+        }
+        if constexpr (kk == 3 && i < 3) fa_k_read<NL, i>(w);
+        // the last two operand blocks, then the next tile's scores
+        if constexpr (kk == 0 && i < 13) fa_softmax<NL, 38 + i>(w);
+        if constexpr ((kk == 1 || kk == 2) && i % 2 == 1) fa_take<NL, 8 * (kk - 1) + i / 2>(w);
+        if constexpr (kk == 3 && i == 3) w.tmax = pair_max(w.tmax);
+        if constexpr (kk == 3 && i == 5) raise = __builtin_amdgcn_ballot_w64(w.tmax > w.mref + kFaSlack);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
+  }
+  // no read or load of this wave is in flight when its registers and the
+  // workgroup's LDS are given back
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    fa_settle(w.ka[i][0]);
+    fa_settle(w.ka[i][1]);
+  }
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void attn_prefill_mfma_kernel(
+    QhAttnPrefillParams p) {
+#ifdef __HIP_DEVICE_COMPILE__
+  extern __shared__ __align__(1024) uint8_t smem[];
   // the last query blocks (the most tiles) are dispatched first
   const int kvh = blockIdx.x, m0 = (gridDim.y - 1 - blockIdx.y) * 32;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, h = lane >> 5;
   const int head = kvh * 4 + wid;
-  const int qpos = p.past + m0 + r;      // its position
   const int kv_end = p.past + min(m0 + 32, p.M);
-  const int q0pos = p.past + m0;         // the workgroup's first query position
   const uint16_t* kbase = p.k_cache + (size_t)kvh * p.max_seq * 256;
   const uint16_t* vbase = p.v_cache + (size_t)kvh * p.max_seq * 256;
 
-  // K / V rows of this KV head through range-checked buffer resources: rows
-  // at or past kv_end read as zeros, so the tile loads carry no branch
-  const auto rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kbase), (short)0, kv_end * 512,
-                                                    0x00020000);
-  const auto rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(vbase), (short)0, kv_end * 512,
-                                                    0x00020000);
-  // K: 64 rows x 32 chunks of 16 bytes, chunk tid + 256 i (coalesced).
-  // V: thread (pg, dc) = (tid % 8, tid / 8) takes positions 8 pg .. + 7 of
-  // dimensions 8 dc .. + 7 and stores them transposed.
-  const int pg = tid & 7, dc = tid >> 3;
-  u32x4 kv[8], vv[8];
-  auto load_k = [&](int t0) {
+  // K / V rows of this KV head through range-checked buffer resources that
+  // start at the tile: rows at or past kv_end read as zeros (past the last
+  // tile all do, without memory traffic), so the tile loads carry no branch.
+  // Load i of a wave fills rows 16 wid + 2 i and + 1 of the stage, lane l slot
+  // l % 32 of row l / 32; an immediate offset counts for the memory and the
+  // LDS address alike.
+  uint32_t ko[8], vo[4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int c = tid + 256 * i;
-      kv[i] = __builtin_amdgcn_raw_buffer_load_b128(rk, (uint32_t)((t0 + (c >> 5)) * 512 + (c & 31) * 16), 0, 0);
-    }
-  };
-  auto load_v = [&](int t0) {
+  for (int i = 0; i < 8; ++i)
+    ko[i] = (uint32_t)((16 * wid + h + 8 * (i / 4)) * 512 + 16 * (r ^ (2 * i + h)));
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      vv[i] = __builtin_amdgcn_raw_buffer_load_b128(rv, (uint32_t)((t0 + 8 * pg + i) * 512 + dc * 16), 0, 0);
+  for (int i = 0; i < 4; ++i)
+    vo[i] = (uint32_t)((16 * wid + h + 8 * (i / 2)) * 512 + 16 * (r ^ (4 * ((2 * i + h) & 3))));
+  // The workgroups that one XCD runs at a time (32 of every second block, see
+  // the grid) start at tiles spread over the unmasked ones and wrap around:
+  // in lockstep from tile 0, each tile was a miss of the XCD's L2 for all of
+  // them at once (3700 tokens: 193 us against 182).
+  const int nt = (kv_end + kFaTile - 1) / kFaTile, tmask = (p.past + m0 + 1) / kFaTile;
+  const int first = __builtin_amdgcn_readfirstlane((int)((blockIdx.y / 2) & 31) * tmask / 32);
+  auto at = [&](int t) { return t + first - (t + first >= nt ? nt : 0); };
+  auto tile_of = [&](const uint16_t* base, int t) {
+    const int tile = at(t);
+    const int left = t < nt ? min(kv_end - tile * kFaTile, kFaTile) * 512 : 0;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base + (size_t)tile * (kFaTile * 256)), (short)0,
+                                             __builtin_amdgcn_readfirstlane(left), 0x00020000);
   };
-  load_k(0);
-  load_v(0);
+  auto issue_k = [&](int t) {
+    uint8_t* stage = smem + (t & 1) * kFaStage + wid * 8192;
+    const auto rk = tile_of(kbase, t);
+    fa_for<8>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (fa_lds_ptr)(stage + 4096 * (i / 4)), 16, ko[i], 0, 1024 * (i % 4), 0);
+    });
+  };
+  auto issue_v = [&](int t) {
+    uint8_t* stage = smem + kFaV0 + (t & 1) * kFaStage + wid * 8192;
+    const auto rv = tile_of(vbase, t);
+    fa_for<8>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (fa_lds_ptr)(stage + 4096 * (i / 4)), 16, vo[2 * (i / 4) + i % 2], 0,
+                                               1024 * (i % 4), 0);
+    });
+  };
 
-  // Q^T operand: dims 16 kk + 8 h .. + 7 of the lane's query, hi in
-  // registers, lo in this wave's LDS rows.  The wave loads its 32 query rows
-  // coalesced (row i by all 64 lanes, 4 dimensions each), splits them, and
-  // hands the hi parts to the lanes that own them through the K / V area,
-  // which is free until the first tile is stored.
-  u32x4 qhi[16];
+  // Q^T operands: dims 16 kk + 8 h .. + 7 of the lane's query.  The wave loads
+  // its 32 query rows coalesced (row i by all 64 lanes, 4 dimensions each),
+  // splits them, and hands first the hi and then the lo parts to the lanes
+  // that own them through its quarter of the V stages (8-byte pieces, the
+  // 16-byte slots swizzled by row as in the K tiles).
+  u32x4 qhi[16], qlo[16];
   uint32_t lo_mask = 0;  // 16-dimension blocks whose lo part is nonzero in this wave
-  uint8_t* sQw = smem + kFaQ0 + wid * 32 * kFaQRow;
-  uint8_t* sHw = smem + wid * 32 * kFaQRow;  // 4 x 16,896 B, below kFaQ0
-  uint8_t* sQ = sQw + r * kFaQRow + 16 * h;
   {
     float4 qa[32];
 #pragma unroll
     for (int i = 0; i < 32; ++i)
       qa[i] = *(const float4*)(p.q + ((size_t)min(m0 + i, p.M - 1) * p.Hq + head) * 256 + 4 * lane);
     __builtin_amdgcn_sched_barrier(0);
-    uint64_t nzl = 0;
+    issue_k(0);
+    issue_k(1);
+    uint8_t* sx = smem + kFaV0 + wid * 16384;
+    uint32_t nz = 0;
+    u32x2 lo[32];
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
       const float v[4] = {qa[i].x * 0.0625f, qa[i].y * 0.0625f, qa[i].z * 0.0625f, qa[i].w * 0.0625f};
-      u32x2 hi, lo;
+      u32x2 hi;
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
-        const float ah = rbf(v[2 * q]), bh = rbf(v[2 * q + 1]);
-        hi[q] = (__float_as_uint(ah) >> 16) | (__float_as_uint(bh) & 0xFFFF0000u);
-        lo[q] = pack_bf2(v[2 * q] - ah, v[2 * q + 1] - bh);
+        hi[q] = pack_pair(v[2 * q], v[2 * q + 1]);
+        lo[i][q] = pack_pair(v[2 * q] - bf_lo(hi[q]), v[2 * q + 1] - bf_hi(hi[q]));
       }
-      *(u32x2*)(sHw + i * kFaQRow + 8 * lane) = hi;
-      *(u32x2*)(sQw + i * kFaQRow + 8 * lane) = lo;
-      nzl |= __builtin_amdgcn_ballot_w64((lo.x | lo.y) != 0u);
+      *(u32x2*)(sx + i * 512 + 16 * ((lane >> 1) ^ (i & 15)) + 8 * (lane & 1)) = hi;
+      nz |= lo[i].x | lo[i].y;
     }
+    const uint64_t nzl = __builtin_amdgcn_ballot_w64(nz != 0u);
 #pragma unroll
     for (int kk = 0; kk < 16; ++kk)
       if ((nzl >> (4 * kk)) & 0xFu) lo_mask |= 1u << kk;
-    __syncthreads();
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) qhi[kk] = *(const u32x4*)(sHw + r * kFaQRow + 32 * kk + 16 * h);
+    for (int kk = 0; kk < 16; ++kk) qhi[kk] = *(const u32x4*)(sx + r * 512 + 16 * ((2 * kk + h) ^ (r & 15)));
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 32; ++i)
+      *(u32x2*)(sx + i * 512 + 16 * ((lane >> 1) ^ (i & 15)) + 8 * (lane & 1)) = lo[i];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk) qlo[kk] = *(const u32x4*)(sx + r * 512 + 16 * ((2 * kk + h) ^ (r & 15)));
   }
-  // lo terms for blocks 0 .. nlo - 1, four at a time (a block whose lo is
-  // zero adds zero)
-  const int nlo = lo_mask ? 32 - __builtin_clz(lo_mask) : 0;
-  v16f_fa o[8];
-#pragma unroll
-  for (int d = 0; d < 8; ++d)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) o[d][e] = 0.0f;
-  float mref = -INFINITY, lrow = 0.0f;
+  __syncthreads();  // the exchange is over
+  issue_v(0);
+  issue_v(1);
 
-  const uint8_t* ka_row = sK + r * kFaKRow + 16 * h;
-  for (int t0 = 0; t0 < kv_end; t0 += kFaTile) {
-    __syncthreads();  // every wave is done with the previous tile
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(fa_lds_ptr)smem;
+  auto run = [&](auto& w, auto nl) {
+    constexpr int NL = decltype(nl)::value;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int c = tid + 256 * i;
-      *(u32x4*)(sK + (c >> 5) * kFaKRow + (c & 31) * 16) = kv[i];
-    }
-    // V^T row 8 dc + j, positions 8 pg .. + 7: pairs of 16-bit halves
+    for (int kk = 0; kk < 16; ++kk) w.qhi[kk] = qhi[kk];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
-      u32x4 col;
+    for (int kk = 0; kk < NL; ++kk) w.qlo[kk] = qlo[kk];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) col[q] = __builtin_amdgcn_perm(vv[2 * q + 1][j >> 1], vv[2 * q][j >> 1], sel);
-      *(u32x4*)(sV + (8 * dc + j) * kFaVRow + 16 * pg) = col;
-    }
-    __syncthreads();
-    load_k(t0 + kFaTile);  // past kv_end: zeros, no memory traffic
-
-    // S^T for the two 32-position blocks (two independent chains; four, with
-    // the even and odd blocks summed afterwards, measured slower: 3.7 k ->
-    // 4.0 k cycles per tile)
-    v16f_fa s0, s1;
+    for (int i = 0; i < 8; ++i) w.kaddr[i] = lds0 + (uint32_t)(r * 512 + 16 * ((2 * i + h) ^ (r & 15)));
+    const int rr = (lane >> 2) & 3;  // row of the 4 x 16 block this lane reads
 #pragma unroll
-    for (int e = 0; e < 16; ++e) s0[e] = s1[e] = 0.0f;
+    for (int i = 0; i < 4; ++i)
+      w.vaddr[i] = lds0 + (uint32_t)(kFaV0 + (4 * h + rr) * 512 + 64 * (i ^ rr) + 32 * ((lane >> 4) & 1) + 8 * (lane & 3));
+    w.lim = p.past + m0 + r - 4 * h;
+    fa_tiles<NL>(w, nt, tmask, at, issue_k, issue_v);
+    // out = bf16(bf16(O / l) * bf16(sigmoid(gate))): O / l goes through LDS, so
+    // that a wave reads its gates and writes its results in whole rows (a lane's
+    // own 8-byte pieces of 32 rows took about 7 us of each workgroup's time).
+    u32x2 gw[32];
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      const v8bf_fa ka0 = __builtin_bit_cast(v8bf_fa, *(const u32x4*)(ka_row + 32 * kk));
-      const v8bf_fa ka1 = __builtin_bit_cast(v8bf_fa, *(const u32x4*)(ka_row + 32 * kFaKRow + 32 * kk));
-      const v8bf_fa qb = __builtin_bit_cast(v8bf_fa, qhi[kk]);
-      s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka0, qb, s0, 0, 0, 0);
-      s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka1, qb, s1, 0, 0, 0);
-    }
-    for (int g = 0; g < nlo; g += 4) {
+    for (int i = 0; i < 32; ++i)
+      gw[i] = *(const u32x2*)(p.gate + (size_t)min(m0 + i, p.M - 1) * p.gate_mstride + (size_t)head * p.gate_hstride +
+                              4 * lane);
+    const float inv = 1.0f / pair_sum(w.lsum);
+    __syncthreads();  // every wave is done with the K / V stages
+    uint8_t* so = smem + wid * 32768;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int kk = g + i;
-        const v8bf_fa ka0 = __builtin_bit_cast(v8bf_fa, *(const u32x4*)(ka_row + 32 * kk));
-        const v8bf_fa ka1 = __builtin_bit_cast(v8bf_fa, *(const u32x4*)(ka_row + 32 * kFaKRow + 32 * kk));
-        const v8bf_fa ql = __builtin_bit_cast(v8bf_fa, *(const u32x4*)(sQ + 32 * kk));
-        s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka0, ql, s0, 0, 0, 0);
-        s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka1, ql, s1, 0, 0, 0);
+    for (int d = 0; d < 8; ++d)
+#pragma unroll
+      for (int b4 = 0; b4 < 4; ++b4) {
+        f32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = w.o[d][4 * b4 + i] * inv;
+        *(f32x4*)(so + r * 1024 + 16 * ((8 * d + 2 * b4 + h) ^ (r & 15))) = v;
       }
+    __builtin_amdgcn_wave_barrier();
+    uint16_t* dst = p.out + (size_t)m0 * p.Hq * 256 + (size_t)head * 256 + 4 * lane;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      if (m0 + i >= p.M) break;
+      const f32x4 v = *(const f32x4*)(so + i * 1024 + 16 * (lane ^ (i & 15)));
+      const uint32_t a = pack_pair(v.x, v.y), b = pack_pair(v.z, v.w);
+      const uint32_t s0 = pack_pair(qh_sigmoid_bf(bf_lo(gw[i].x)), qh_sigmoid_bf(bf_hi(gw[i].x)));
+      const uint32_t s1 = pack_pair(qh_sigmoid_bf(bf_lo(gw[i].y)), qh_sigmoid_bf(bf_hi(gw[i].y)));
+      *(u32x2*)(dst + (size_t)i * p.Hq * 256) =
+          u32x2{pack_pair(bf_lo(a) * bf_lo(s0), bf_hi(a) * bf_hi(s0)), pack_pair(bf_lo(b) * bf_lo(s1), bf_hi(b) * bf_hi(s1))};
     }
-    // causal mask on tiles that reach past the first query position: score
-    // e of block nt is position t0 + 32 nt + 8 (e / 4) + 4 h + e % 4
-    if (t0 + kFaTile - 1 > q0pos) {
-      const int lim = qpos - t0 - 4 * h;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int idx = 8 * (e >> 2) + (e & 3);
-        s0[e] = idx <= lim ? s0[e] : -INFINITY;
-        s1[e] = idx + 32 <= lim ? s1[e] : -INFINITY;
-      }
-    }
-    float tmax = fmaxf(s0[0], s1[0]);
-#pragma unroll
-    for (int e = 1; e < 16; ++e) tmax = fmaxf(tmax, fmaxf(s0[e], s1[e]));
-    tmax = pair_max(tmax);
-    if (__builtin_amdgcn_ballot_w64(tmax > mref + kFaSlack) != 0) {
-      // every row's first tile has position 0 unmasked, so mnew is finite
-      const float mnew = fmaxf(mref, tmax);
-      const float corr = mnew == mref ? 1.0f : __expf(mref - mnew);
-      lrow *= corr;
-#pragma unroll
-      for (int d = 0; d < 8; ++d)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          float x = o[d][e], t;
-          asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32_e32 %1, %2, %1\n\tv_accvgpr_write_b32 %0, %1"
-                       : "+a"(x), "=&v"(t)
-                       : "v"(corr));
-          o[d][e] = x;
-        }
-      mref = mnew;
-    }
-    float psum = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      s0[e] = __expf(s0[e] - mref);
-      s1[e] = __expf(s1[e] - mref);
-      psum += s0[e] + s1[e];
-    }
-    lrow += pair_sum(psum);
-    // P^T operand of block kk: positions 16 kk + 8 h .. + 7 of the lane's
-    // row.  Lane h = 0 holds positions 0-3 and 8-11 of each 16, lane h = 1
-    // positions 4-7 and 12-15; one swap of the middle pair gives both lanes
-    // their 8 in order.
-    u32x4 phi[4], plo[4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const v16f_fa& sv = kk < 2 ? s0 : s1;
-      const int b = 8 * (kk & 1);
-      float v[8];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(sv[b + i]), __float_as_uint(sv[b + 4 + i]),
-                                                         false, false);
-        v[i] = __uint_as_float(sw[0]);
-        v[4 + i] = __uint_as_float(sw[1]);
-      }
-      split8(v, phi[kk], plo[kk]);
-    }
-    load_v(t0 + kFaTile);
-    // O^T += V^T P^T over 8 blocks of 32 dimensions; consecutive products
-    // go to different accumulators
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      v8bf_fa va[8];
-#pragma unroll
-      for (int d = 0; d < 8; ++d)
-        va[d] = __builtin_bit_cast(v8bf_fa, *(const u32x4*)(sV + (32 * d + r) * kFaVRow + 16 * h + 32 * kk));
-#pragma unroll
-      for (int d = 0; d < 8; ++d)
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[d], __builtin_bit_cast(v8bf_fa, phi[kk]), o[d], 0, 0, 0);
-#pragma unroll
-      for (int d = 0; d < 8; ++d)
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[d], __builtin_bit_cast(v8bf_fa, plo[kk]), o[d], 0, 0, 0);
-    }
+  };
+  if (lo_mask >> 4) {
+    FaWave<16> w;
+    run(w, std::integral_constant<int, 16>{});
+  } else {
+    FaWave<4> w;
+    run(w, std::integral_constant<int, 4>{});
   }
-  // out = bf16(bf16(O / l) * bf16(sigmoid(gate))) for the lane's query
-  if (m0 + r >= p.M) return;
-  const float inv = 1.0f / lrow;
-  const uint16_t* gp = p.gate + (size_t)(m0 + r) * p.gate_mstride + (size_t)head * p.gate_hstride;
-  uint16_t* dst = p.out + (size_t)(m0 + r) * p.Hq * 256 + (size_t)head * 256;
-#pragma unroll
-  for (int d = 0; d < 8; ++d)
-#pragma unroll
-    for (int b4 = 0; b4 < 4; ++b4) {
-      const int dim = 32 * d + 8 * b4 + 4 * h;
-      const u32x2 gw = *(const u32x2*)(gp + dim);
-      const float g[4] = {bf_lo(gw.x), bf_hi(gw.x), bf_lo(gw.y), bf_hi(gw.y)};
-      float y[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = rbf(o[d][4 * b4 + i] * inv) * rbf(qh_sigmoid(g[i]));
-      *(u32x2*)(dst + dim) = u32x2{pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3])};
-    }
+#endif
 }
 
 // ---- GDN conv over the sequence: one thread per (token, channel) -------------
@@ -913,12 +1134,14 @@ int qh_launch_attn_prefill(const QhAttnPrefillParams& p, hipStream_t st) {
     return -1;
   }
   if (p.M <= 0) return 0;
-  // D = 256 with 4 query heads per KV head, 16-byte aligned rows and at
-  // least 256 tokens: the matrix-core kernel (one workgroup per 32 tokens);
-  // other launches the per-token one.  Measured per layer at 4 KV heads:
-  // 128 tokens 15.3 vs 27.5 us, 256 tokens 38 vs 38 us, 512 tokens 116 vs
-  // 54 us, 3700 tokens 4.3 ms vs 0.45 ms (per-token vs matrix-core).
-  if (p.M >= 256 && p.D == 256 && p.Hq == 4 * p.Hkv && (uintptr_t)p.q % 16 == 0 && (uintptr_t)p.gate % 8 == 0 &&
+  // D = 256 with 4 query heads per KV head, 16-byte aligned rows and a last
+  // token that sees at least 256 positions: the matrix-core kernel (one
+  // workgroup per 32 tokens); other launches the per-token one.  A workgroup of
+  // the first takes 18 us and 2.0 us per 64 positions, one of the second 3 us
+  // and 2.6 us per 32 positions.  Measured per layer at 4 KV heads, per-token
+  // vs matrix-core: 128 tokens 14 vs 22 us, 224 tokens 28.5 vs 26 us, 128
+  // tokens after 1000 118 vs 54 us, 128 after 3000 304 vs 117 us.
+  if (p.past + p.M >= 256 && p.D == 256 && p.Hq == 4 * p.Hkv && (uintptr_t)p.q % 16 == 0 && (uintptr_t)p.gate % 8 == 0 &&
       p.gate_mstride % 4 == 0 && p.gate_hstride % 4 == 0 && (uintptr_t)p.k_cache % 16 == 0 &&
       (uintptr_t)p.v_cache % 16 == 0 && (uintptr_t)p.out % 8 == 0) {
     hipLaunchKernelGGL(attn_prefill_mfma_kernel, dim3(p.Hkv, (p.M + 31) / 32), dim3(256), (size_t)kFaLds, st, p);

@@ -227,6 +227,21 @@ __device__ __forceinline__ float qh_silu_bf(float x) {
   const float y = fmaf(fmaf(-q, d, x), __builtin_amdgcn_rcpf(d), q);
   return x > 88.0f ? x : y;
 }
+// Sigmoid of a bf16 value whose result is rounded to bf16, by the same steps:
+// e^-x corrected to first order, one Newton step on the hardware reciprocal.
+// Above 88 it is 1; where the result would be denormal (below -87.3) zero; NaN
+// stays NaN.  For all other bf16 arguments it rounds to the bf16 value that
+// 64-bit arithmetic gives (test_attention_gate_every_argument).
+__device__ __forceinline__ float qh_sigmoid_bf(float x) {
+  const float a = x < -88.0f ? 88.0f : x > 88.0f ? -88.0f : -x;
+  const float t = a * 1.44269502f;
+  const float c = fmaf(a, 1.92596299e-8f, fmaf(a, 1.44269502f, -t));
+  const float e = __builtin_amdgcn_exp2f(t);
+  const float d = 1.0f + fmaf(e, c * 0.693147182f, e);
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float y = fmaf(fmaf(-r, d, 1.0f), r, r);
+  return x < -88.0f ? 0.0f : y;
+}
 // SiLU on the fast exponential, for per-element loops on a kernel's critical
 // path (the gated RMSNorm prologue of the decode output projection).
 // The reciprocal is the hardware v_rcp_f32 (about 1 ulp) in place of the IEEE

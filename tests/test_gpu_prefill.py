@@ -23,9 +23,9 @@ def cu(t):
 
 
 # (tokens, past): positions 0 .. past-1 are cached by an earlier prep call,
-# positions past .. tokens-1 are the prefill.  Prefills of 256 or more tokens
-# run the matrix-core kernel (300: a ragged last 32-token block; 330 - 70 =
-# 260 after a cached prefix), shorter ones the per-token kernel.
+# positions past .. tokens-1 are the prefill.  From 256 positions on the
+# matrix-core kernel runs (300: a ragged last 32-token block; 330 - 70 =
+# 260 after a cached prefix), below that the per-token kernel.
 # The last two cases take the per-token kernel with two query heads per wave
 # (8 per KV head, head dim 128) and with an idle wave (3 per KV head).
 @pytest.mark.parametrize("M,past,Hq,Hkv,D", [(37, 0, 8, 2, 256), (70, 0, 8, 2, 256), (100, 20, 8, 2, 256),
@@ -76,6 +76,64 @@ def test_attention_prefill(M, past, Hq, Hkv, D):
         ref[:, h] = orc.bf16(torch.softmax(sc, dim=-1) @ V[kv])
     ref = orc.bf16(ref.reshape(M, -1) * orc.bf16(torch.sigmoid(q_all[..., D:].float().reshape(M, -1))))
     assert_close(out, ref[past:], atol_frac=1e-3, what="prefill attention")
+
+
+# Matrix-core attention at its edges against float64 on the host: one query row
+# after a prefix, one past a tile and past a 32-token block, several row blocks
+# whose tile order starts at different tiles, and queries with a low part in
+# every dimension (rot 256: all 16 blocks of the split q are computed).  The
+# kernel's own q and caches are the input, so that only its arithmetic is
+# measured: three roundings to bf16 (attention, sigmoid, their product) of at most
+# 2^-8 relative each (8 significant bits: half an ulp of a value just above a
+# power of two), and 2^-16 per operand from the split q and p.
+@pytest.mark.parametrize("M,past,Hkv,split_all", [(1, 255, 2, False), (5, 251, 1, True), (33, 256, 2, False),
+                                                  (257, 0, 1, True), (65, 700, 2, False), (200, 1848, 1, False)])
+def test_attention_prefill_matrix_cores(M, past, Hkv, split_all):
+    g = gen(5 + M)
+    D, Hq, max_seq = 256, 4 * Hkv, 2048
+    q = randn(g, M, Hq, D)
+    if not split_all:
+        q[..., 64:] = bf(q[..., 64:]).float()
+    kc, vc = bf(randn(g, Hkv, max_seq, D)), bf(randn(g, Hkv, max_seq, D))
+    kc[:, past + M:], vc[:, past + M:] = float("nan"), float("nan")  # rows no query may see
+    gate = bf(randn(g, M, Hq, D))
+    out = torch.empty(M, Hq * D, dtype=torch.bfloat16, device=DEV)
+    dq, dg, dk, dv = cu(q), cu(gate), cu(kc), cu(vc)
+    lib = abi.load()
+    abi.check(lib.qh_attn_prefill(abi.ptr(dq), abi.ptr(dg), Hq * D, D, abi.ptr(dk), abi.ptr(dv), abi.ptr(out), M,
+                                  Hq, Hkv, D, past, max_seq, abi.stream_handle()))
+    torch.cuda.synchronize()
+    end = past + M
+    mask = torch.arange(end)[None, :] > torch.arange(past, end)[:, None]
+    ref = torch.empty(M, Hq, D, dtype=torch.float64)
+    for h in range(Hq):
+        sc = (q[:, h].double() @ kc[h // 4, :end].double().t()) / 16.0
+        ref[:, h] = torch.softmax(sc.masked_fill(mask, -math.inf), -1) @ vc[h // 4, :end].double()
+    ref = (ref * torch.sigmoid(gate.double())).reshape(M, -1)
+    assert_close(out, ref.float(), rtol=3 * 2 ** -8 + 2 ** -12, atol_frac=2 ** -14, what="matrix-core attention")
+
+
+# Every bf16 gate: with zero keys and values of one, attention is one and the
+# output is bf16(sigmoid(gate)).  The kernel's sigmoid rounds to the value that
+# 64-bit arithmetic gives; results below the smallest normal number, 2^-126
+# (gates below -87.3), are zero.
+def test_attention_gate_every_argument():
+    M, Hq, Hkv, D = 256, 4, 1, 256
+    gate = torch.arange(M * Hq * D, dtype=torch.int32).remainder(65536).to(torch.uint16).view(torch.bfloat16)
+    q = torch.zeros(M, Hq, D, device=DEV)
+    kc = torch.zeros(Hkv, M, D, dtype=torch.bfloat16, device=DEV)
+    vc, dg = torch.ones_like(kc), gate.cuda()
+    out = torch.empty(M, Hq * D, dtype=torch.bfloat16, device=DEV)
+    lib = abi.load()
+    abi.check(lib.qh_attn_prefill(abi.ptr(q), abi.ptr(dg), Hq * D, D, abi.ptr(kc), abi.ptr(vc), abi.ptr(out), M, Hq,
+                                  Hkv, D, 0, M, abi.stream_handle()))
+    torch.cuda.synchronize()
+    got, x = out.view(-1)[:65536].cpu(), gate[:65536]
+    assert torch.equal(got.isnan(), x.isnan())
+    want = torch.sigmoid(x.double()).to(torch.bfloat16)
+    normal = want.float() >= 2.0 ** -126
+    assert torch.equal(got[normal], want[normal])
+    assert (got[~normal & ~x.isnan()] == 0).all()
 
 
 # M = 45: five full 8-token blocks of the scan plus a tail; M = 3: fewer
