@@ -78,6 +78,31 @@ def test_attention_prefill(M, past, Hq, Hkv, D):
     assert_close(out, ref[past:], atol_frac=1e-3, what="prefill attention")
 
 
+# The vector head-norm kernel (four rows per wave from 8192 rows on: 823 tokens x
+# 10 rows, no multiple of its 16 rows a workgroup; else one) against the general
+# one, which a q output 4 bytes off takes: the same arithmetic, the same bits.
+@pytest.mark.parametrize("M,past,rot,norm", [(823, 0, 64, True), (823, 9, 256, True), (7, 3, 64, True),
+                                             (1, 0, 8, False), (823, 0, 0, False)])
+def test_attention_prep_vector_rows(M, past, rot, norm):
+    g = gen(31 + M + rot)
+    Hq, Hkv, D, max_seq = 8, 2, 256, 840
+    q, k, v = cu(bf(randn(g, M, Hq, 2 * D))), cu(bf(randn(g, M, Hkv, D))), cu(bf(randn(g, M, Hkv, D)))
+    qn, kn = cu(randn(g, D, std=0.1)), cu(randn(g, D, std=0.1))
+    cos, sin = (cu(t) for t in orc.rope_tables(max_seq, max(rot, 2), 1e7))
+    lib, got = abi.load(), []
+    for off in (0, 1):
+        q32 = torch.zeros(M * Hq * D + off, device=DEV)[off:]
+        kc = torch.zeros(Hkv, max_seq, D, dtype=torch.bfloat16, device=DEV)
+        vc = torch.zeros_like(kc)
+        abi.check(lib.qh_attn_prep(abi.ptr(q), abi.ptr(k), abi.ptr(v), abi.ptr(qn) if norm else None,
+                                   abi.ptr(kn) if norm else None, abi.ptr(cos), abi.ptr(sin), abi.ptr(q32),
+                                   abi.ptr(kc), abi.ptr(vc), M, Hq, Hkv, D, rot, past, max_seq, 1e-6,
+                                   abi.stream_handle()))
+        got.append((q32, kc, vc))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 # Matrix-core attention at its edges against float64 on the host: one query row
 # after a prefix, one past a tile and past a 32-token block, several row blocks
 # whose tile order starts at different tiles, and queries with a low part in
