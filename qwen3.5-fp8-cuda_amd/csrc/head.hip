@@ -68,8 +68,8 @@ void launch(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int N, int
 }  // namespace
 
 int qh_launch_head_rows(const void* x, const void* w, void* logits, int M, int N, int K, hipStream_t st) {
-  // the tiles' buffer ranges (128 rows of K bf16) stay below 2^31 bytes
-  if (K <= 0 || K % 64 != 0 || K > (1 << 22) || (uintptr_t)x % 16 != 0 || (uintptr_t)w % 16 != 0) {
+  // the tiles' buffer ranges (up to 256 rows of K bf16) stay below 2^31 bytes
+  if (K <= 0 || K % 64 != 0 || K >= (1 << 22) || (uintptr_t)x % 16 != 0 || (uintptr_t)w % 16 != 0) {
     qh_set_error("lm_head rows: K=%d must be a positive multiple of 64, x and w 16-byte aligned", K);
     return -1;
   }
