@@ -1040,8 +1040,8 @@ inline long tiles_of(const QhGemmSeg* seg, int nseg, int bn) {
 //    replaces the add + norm launch that would follow.
 //  - Ring kernel beside it where its model holds and the tile shapes leave
 //    CUs idle: one 64 x 64 tile per CU (1024 x 1024 x 2560: 15.4 us against
-//    17.9), one round of 64 x 128 at two workgroups per CU (400 x 8192 x 2560:
-//    27.3 against 30.4).  Every other ring plan lost (3700 x 18432 x 2560: 387
+//    17.9), one or two rounds of 64 x 128 at two workgroups per CU (400 x 8192 x
+//    2560: 27.3 against 30.4; 416 x 18432 x 2560: 53.4 against 58.7).  Every other ring plan lost (3700 x 18432 x 2560: 387
 //    against 346 us; 24 x 2560 x 9216: 48 against 12).
 //  - Other scale modes: the ring kernel's own plans (gemm_plan_ring).
 GemmPlan gemm_plan_ring(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const void* ws, size_t ws_bytes);
@@ -1059,8 +1059,9 @@ GemmPlan gemm_plan(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const 
   double best_t = 1e300;
   const long r64 = (long)((M + 63) / 64) * tiles_of(seg, nseg, 64), r128 = (long)((M + 63) / 64) * tiles_of(seg, nseg, 128);
   if (r64 <= cus) best_t = 2.8 + 0.61 * KB;
-  if (r128 > cus && r128 <= 2L * cus && 5.39 + 1.06 * KB < best_t) {
-    best_t = 5.39 + 1.06 * KB;
+  const double t128 = (double)((r128 + 2L * cus - 1) / (2L * cus)) * (5.39 + 1.06 * KB);
+  if (r128 > cus && r128 <= 4L * cus && t128 < best_t) {
+    best_t = t128;
     best = {-1, 64, 128, 2, 128, 1, 0};
   }
   for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
