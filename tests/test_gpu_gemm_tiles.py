@@ -42,6 +42,7 @@ def check(y, ref, mag, K, what):
     (137, 13615, 256), (635, 4513, 256), (2490, 1595, 384),             # 128 x 160
     (281, 13694, 256), (815, 7373, 512),                                # 128 x 256
     (391, 18067, 256), (943, 8514, 384),                                # 128 x 320
+    (389, 18401, 2560), (448, 18432, 2560),                             # ring, two rounds of 64 x 128
     (5, 300, 16384), (5, 300, 16512),                                   # 128 K blocks, and one more (ring kernel)
 ])
 def test_gemm_tile_shapes(M, N, K):
