@@ -870,18 +870,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_tile_kernel(const uint16_t
     float* pz = part + ((size_t)z * M + m0) * ldp + (size_t)tn * nstep;
     qh_tile::finish<C>(t, smem, acc, [&](int m, int n, f32x4 v) { *(f32x4*)(pz + (size_t)m * ldp + n) = v; });
   } else {
-    uint16_t* y = g.y[si] + (size_t)m0 * N + n0;
-    const bool vec = N % 4 == 0 && (uintptr_t)g.y[si] % 8 == 0;
-    qh_tile::finish<C>(t, smem, acc, [&](int m, int n, f32x4 v) {
-      uint16_t* dst = y + (size_t)m * N + n;
-      if (vec) {
-        *(u32x2*)dst = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
-      } else {
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          if (n + c < t.rows_n) dst[c] = f2bf(v[c]);
-      }
-    });
+    qh_tile::store_rows<C>(t, smem, acc, g.y[si] + (size_t)m0 * N + n0, N);
   }
 }
 

@@ -337,4 +337,92 @@ __device__ __forceinline__ void finish(const Work& t, uint8_t* smem, f32x4 (&acc
   }
 }
 
+// Rows first, first + step, .. < n of a wave's sub-tile (LR elements apart in
+// LDS) to y: ld(row) reads the lane's value, put(row pointer, value) stores it.
+// Eight reads ahead of their stores.
+template <typename L, typename P>
+__device__ __forceinline__ void copy_rows(int first, int step, int n, uint16_t* y, int ldy, L ld, P put) {
+  int i = first;
+  for (; i + 7 * step < n; i += 8 * step) {
+    uint32_t v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = ld(i + k * step);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) put(y + (size_t)(i + k * step) * ldy, v[k]);
+  }
+  for (; i < n; i += step) put(y + (size_t)i * ldy, ld(i));
+}
+
+// The tile as bf16 rows of y (the tile's first element; row stride ldy).  Rows
+// whose 4-column groups are 8-byte aligned take one store per group straight
+// from the accumulators.  Other rows (ldy % 4 != 0) would need four 2-byte
+// stores per group, each over 16 rows of 32 bytes; with one or two K groups
+// each wave turns its sub-tile into rows through LDS instead and stores
+// aligned pairs of columns, consecutive lanes consecutive pairs, with the
+// lanes chosen once for all rows that start on an odd element and once for the
+// others: a lone wave issues an instruction per 5 cycles, so a test per row
+// costs as much as the stores.  3153 x 5003 x 640 on 128 x 256 tiles: 48.0 us
+// with 2-byte stores, 44 with a test per row, 34.9 now (5004 columns: 29.5);
+// 3153 x 5003 x 2560: 96 -> 85 (79).
+template <typename C>
+__device__ __forceinline__ void store_rows(const Work& t, uint8_t* smem, f32x4 (&acc)[C::MI][C::NJ], uint16_t* y,
+                                           int ldy) {
+  const bool vec = ldy % 4 == 0 && (uintptr_t)y % 8 == 0;
+  if constexpr (C::KG <= 2) {
+    if (!vec) {
+      constexpr int W = 16 * C::NJ, LR = W + 4, H = 16 * C::MI;  // the sub-tile, and its row in LDS
+      static_assert((C::KG == 2 ? C::SLAB : 0) + C::GW * H * LR * 2 <= C::LDS && H % 8 == 0, "staged rows");
+      const int lane = threadIdx.x & 63;
+      const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+      const int wm = (wv / C::WN) * H, wn = (wv % C::WN) * W;
+      uint16_t* rows = (uint16_t*)(smem + (C::KG == 2 ? C::SLAB : 0)) + wv * H * LR;
+      if constexpr (C::KG == 1) __syncthreads();  // every wave is done with the ring
+      finish<C>(t, smem, acc, [&](int m, int n, f32x4 v) {
+        *(u32x2*)(rows + (m - wm) * LR + n - wn) = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+      });
+      if (C::KG == 2 && wv >= C::GW) return;
+      const int nr = min(t.rows_m - wm, H), nc = min(t.rows_n - wn, W);
+      if (nr <= 0 || nc <= 0) return;
+      asm volatile("" ::: "memory");  // the wave's own rows, in order through LDS
+      uint16_t* yw = y + (size_t)wm * ldy + wn;
+      const int odd0 = (int)((uintptr_t)yw >> 1) & 1, step = 1 + (ldy & 1);
+      const uint16_t* mine = rows + 2 * min(lane, W / 2);
+      for (int f = 0; f < step; ++f) {
+        if (odd0 ^ f) {  // rows that start on an odd element: pairs (2 lane - 1, 2 lane)
+          if (lane > 0 && 2 * lane < nc)
+            copy_rows(f, step, nr, yw, ldy,
+                      [&](int i) {
+                        const uint16_t* r = mine + i * LR;
+                        return __builtin_amdgcn_alignbyte(*(const uint32_t*)r, *(const uint32_t*)(r - 2), 2);
+                      },
+                      [&](uint16_t* d, uint32_t v) { *(uint32_t*)(d + 2 * lane - 1) = v; });
+          if (lane == 0 || 2 * lane == nc) {  // the first column, and a last one without a partner
+            const int c = lane ? nc - 1 : 0;
+            copy_rows(f, step, nr, yw, ldy, [&](int i) { return (uint32_t)rows[i * LR + c]; },
+                      [&](uint16_t* d, uint32_t v) { d[c] = (uint16_t)v; });
+          }
+        } else {  // pairs (2 lane, 2 lane + 1)
+          if (2 * lane + 1 < nc)
+            copy_rows(f, step, nr, yw, ldy, [&](int i) { return *(const uint32_t*)(mine + i * LR); },
+                      [&](uint16_t* d, uint32_t v) { *(uint32_t*)(d + 2 * lane) = v; });
+          if (2 * lane + 1 == nc)
+            copy_rows(f, step, nr, yw, ldy, [&](int i) { return (uint32_t)rows[i * LR + 2 * lane]; },
+                      [&](uint16_t* d, uint32_t v) { d[2 * lane] = (uint16_t)v; });
+        }
+      }
+      return;
+    }
+  }
+  finish<C>(t, smem, acc, [&](int m, int n, f32x4 v) {
+    uint16_t* d = y + (size_t)m * ldy + n;
+    if (vec) {
+      *(u32x2*)d = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (n + c < t.rows_n) d[c] = f2bf(v[c]);
+    }
+  });
+}
+
 }  // namespace qh_tile

@@ -43,18 +43,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void head_rows_kernel(const uint16_t
   t.u1 = K / C::KU;
   f32x4 acc[C::MI][C::NJ];
   qh_tile::mainloop<C, float>(t, smem, acc);
-  uint16_t* out = y + (size_t)m0 * N + n0;
-  const bool vec = N % 4 == 0 && (uintptr_t)y % 8 == 0;
-  qh_tile::finish<C>(t, smem, acc, [&](int m, int n, f32x4 v) {
-    uint16_t* dst = out + (size_t)m * N + n;
-    if (vec) {
-      *(u32x2*)dst = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
-    } else {
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        if (n + c < t.rows_n) dst[c] = f2bf(v[c]);
-    }
-  });
+  qh_tile::store_rows<C>(t, smem, acc, y + (size_t)m0 * N + n0, N);
 }
 
 template <typename C>

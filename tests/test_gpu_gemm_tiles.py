@@ -57,6 +57,25 @@ def test_gemm_tile_shapes(M, N, K):
         check(y, ref, mag, K, f"{M} x {N} x {K} {scale.dtype}")
 
 
+# Rows that are not 8-byte aligned: every residue of the row stride mod 4, the first element on an
+# odd and on an even 2-byte address, last tiles of one column, an odd and an even number of them.
+# The elements before and after the output stay as they were.
+@pytest.mark.parametrize("M,N,K", [(23, 16851, 640), (25, 16001, 384), (71, 15113, 256), (67, 15842, 256),
+                                   (137, 13615, 256), (130, 13681, 256), (281, 13694, 256), (300, 13057, 384),
+                                   (391, 18067, 256), (389, 17921, 256), (5, 301, 640), (2, 1, 256)])
+@pytest.mark.parametrize("off", [0, 1, 2])
+def test_gemm_tile_unaligned_rows(M, N, K, off):
+    g = gen(M + N + off)
+    w, s = quant(g, N, K)
+    x, dw, ds = bf(randn(g, M, K)), w.to(DEV), s.to(DEV)
+    buf = torch.full((M * N + 16,), 77.0, dtype=torch.bfloat16, device=DEV)
+    y, dx, lib = buf[off:off + M * N], x.to(DEV), abi.load()
+    abi.check(lib.qh_gemm_e4m3(abi.ptr(dx), abi.ptr(dw), abi.ptr(ds), abi.ptr(y), M, N, K, K // 128, 0, None, 0,
+                               abi.stream_handle()), "gemm")
+    check(y.view(M, N), *product(x, w, s), K, f"{M} x {N} x {K} at {off}")
+    assert (buf[:off] == 77.0).all() and (buf[off + M * N:] == 77.0).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(24, 2560, 9216), (128, 2560, 9216), (100, 2500, 4096), (300, 2560, 2560),
                                    (512, 2560, 9216), (2, 12563, 1024), (37, 1001, 9216)])
 def test_gemm_tile_split_k(M, N, K):
