@@ -320,6 +320,13 @@ int qh_gemv_e4m3_gated(const void* core, const void* z, const void* norm_w, int 
  * ws_bytes.  Calls sharing a workspace must not overlap. */
 size_t qh_gemm_workspace_size(int M, int K);
 
+/* How qh_gemm_e4m3* would run nseg projections of N[0 .. nseg - 1] columns in
+ * scale mode kb over M rows on a device of cus CUs, with 16-byte aligned operands
+ * and a workspace of ws_bytes (0: none).  Runs on the host alone.  out[7]: shape of the tile kernel or -1 (ring kernel), tile rows
+ * and columns, workgroups per CU, columns used of a tile, K slices, and the work
+ * items (tile, K slice) per CU of the busiest XCD. */
+int qh_gemm_plan(int M, int K, int nseg, const int* N, int kb, int cus, size_t ws_bytes, int* out);
+
 /* Prefill GEMM on the fp8 matrix cores (fp8_gemm_batch semantics). */
 int qh_gemm_e4m3(const void* x, const void* w, const void* s, void* y, int M, int N, int K,
                  int kb, int scales_bf16, void* ws, size_t ws_bytes, qh_stream_t stream);

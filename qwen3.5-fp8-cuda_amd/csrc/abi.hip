@@ -766,6 +766,15 @@ QH_EXPORT int qh_gated_rmsnorm(const void* core, const void* z, const void* w, v
 
 QH_EXPORT size_t qh_gemm_workspace_size(int M, int K) { return qh_gemm_workspace_bytes(M, K); }
 
+// The launch plan of a prefill GEMM with aligned operands (host only).
+QH_EXPORT int qh_gemm_plan(int M, int K, int nseg, const int* N, int kb, int cus, size_t ws_bytes, int* out) {
+  if (qh_gemm_plan_of(M, K, N, nseg, kb, cus, ws_bytes, out) != 0) {
+    qh_set_error("qh_gemm_plan: M=%d K=%d nseg=%d cus=%d, or a null pointer or segment", M, K, nseg, cus);
+    return -1;
+  }
+  return 0;
+}
+
 // A caller workspace for split-K partials is either absent (ws null: K is not
 // split) or ws_bytes >= qh_gemm_workspace_size bytes, 256-byte aligned.  The
 // check runs before anything touches the device, and the plan never puts more

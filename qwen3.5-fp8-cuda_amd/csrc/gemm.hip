@@ -24,12 +24,10 @@
 //    workgroup, from 16 x 16 with K shared out over eight waves (a few rows) to
 //    128 x 320 (thousands), the shape picked by a time model (gemm_plan);
 //  - gemm_dma_kernel (other scale modes, and where the model favours it):
-//    a 2 x 2 grid of waves per tile; persistent
-//    workgroups stream (tile or tile K slice, K block) units through a
+//    a 2 x 2 grid of waves per tile; persistent workgroups stream (tile or tile K slice, K block) units through a
 //    two-stage LDS ring filled by direct-to-LDS loads, on 64 x 64 tiles
 //    (three workgroups per CU), 64 x 128 (two) or 128 x 192 (one), the plan
-//    (tile shape, K split) picked by a cost model with measured per-unit
-//    cycles (gemm_plan); split-K partials are finished by
+//    (tile shape, K split) picked by a time model too; split-K partials are finished by
 //    gemm_splitk_reduce_kernel or splitk_add_rmsnorm_kernel;
 //  - gemm_e4m3_lds_kernel (fallback for unaligned weights or scales): one
 //    workgroup per (64 x 64 tile, K slice), the next K blocks in registers
@@ -41,6 +39,8 @@
 #include "qh_common.h"
 #include "qh_gemm.h"
 #include "qh_norm.h"
+
+#include <algorithm>
 
 namespace {
 
@@ -639,7 +639,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* pa
                                                                  int ldp, GemmGroup g, int bn);
 
 // reduce = false leaves split-K partials for the caller's own finishing kernel
-// (partial row stride: gemm_part_ldp).
+// (partial row stride: GemmPlan::ldp).
 template <typename ScaleT, int DS, int BN, int BM>
 void launch_gemm_dma(const uint16_t* x, const QhGemmSeg* seg, int nseg, int M, int K, hipStream_t st,
                      int cus, int wpc, int S = 1, float* part = nullptr, bool reduce = true) {
@@ -704,7 +704,7 @@ __device__ __forceinline__ f32x4 sum_slices(const float* p, size_t zs) {
 
 // Split-K finish: y = bf16(sum_z part[z][m][column]), summed in z order;
 // columns past a segment's N (tile padding) are skipped.  Four columns per
-// thread (segments start at multiples of 64 columns).
+// thread (segments start at multiples of bn, itself a multiple of 16).
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* part, int S, int M,
                                                                  int ldp, GemmGroup g, int bn) {
   const size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -970,8 +970,10 @@ namespace {
 // Launch plan: a shape of the tile kernel (tile >= 0: index into kTiles, nstep
 // columns per tile) or of the ring kernel (tile = -1: bm x bn tiles, wpc
 // workgroups per CU), and the K slices S.  ldp: row stride of the partials.
+// load: work items (tile, K slice) per CU of the busiest XCD, as the model counts.
 struct GemmPlan {
   int tile, bm, bn, wpc, nstep, S, ldp;
+  long load;
 };
 
 // Tile kernel shapes: MI, NJ, WM, WN, KG, KU, DS (gemm_tile.h) and whether they
@@ -988,35 +990,66 @@ struct GemmPlan {
   V(8, 4, 4, 2, 4, 1, 128, 2, false)  \
   V(9, 4, 5, 2, 4, 1, 64, 4, false)
 
-// Time model of a launch, in us: a + b (rounds x passes) + c rounds + d (MB a
-// CU pulls in), rounds = ceil(tiles / CUs), passes = K units of one K group.
-// Fitted to 26 row counts (2 .. 3700) x 11 (N, K) (512 x 256 .. 18432 x 2560) on
-// MI355X with the weights out of the caches, rms error 5 - 14 %; over those
-// 286 shapes the plan it picks is 2 % slower than the fastest shape measured.
+// Time model of a launch of the tile kernel, in us:
+//   start + rounds (pass passes + round + x X + w W + odd) + weights nMB + out oMB
+// rounds: tiles on the busiest XCD over its CUs; passes: K units of one K group;
+// X, W: MB of X and of W that a CU takes in for a tile; odd: the share of the
+// columns whose rows are not 8-byte aligned (store_rows); nMB, oMB: MB of weights
+// and of output of the whole launch.  Fitted on MI355X to 4800 (M, N, K) with
+// weights out of the caches (M 2 .. 4096, N 32 .. 18432 in up to four segments,
+// even and odd, K 256 .. 9216), rms error 2 - 5 % a shape.
 struct TileShape {
   int bm, bn, kg, ku;
   bool split;
-  double a, b, c, d;
+  double start, pass, round, x, w, odd, weights, out;
 };
 #define QH_BM(MI, WM) 16 * MI * WM
 #define QH_V(id, MI, NJ, WM, WN, KG, KU, DS, SP) {QH_BM(MI, WM), QH_BM(NJ, WN), KG, KU, SP, QH_TIME_##id},
-#define QH_TIME_0 2.074, 0.2978, 0.9993, 0.5571
-#define QH_TIME_1 0.8717, 0.2865, 2.862, 9.224
-#define QH_TIME_2 0.8305, 0.2711, 2.552, 6.744
-#define QH_TIME_3 0.6686, 0.2669, 3.074, 8.796
-#define QH_TIME_4 1.577, 0.5643, 2.84, 0.6752
-#define QH_TIME_5 0.0, 0.8451, 3.447, 5.105
-#define QH_TIME_6 1.093, 1.245, 3.126, 2.955
-#define QH_TIME_7 0.0, 1.121, 3.915, 2.799
-#define QH_TIME_8 0.0, 1.431, 4.599, 4.072
-#define QH_TIME_9 0.0, 1.113, 5.439, 3.584
+#define QH_TIME_0 2.63, 0.177, 0.575, 5.36, 6.62, 0.055, 0.110, 0.333
+#define QH_TIME_1 0.248, 0.245, 3.42, 5.68, 13.2, 0.028, 0.101, 0.0
+#define QH_TIME_2 1.56, 0.367, 1.85, 2.70, 9.28, 0.051, 0.0956, 0.17
+#define QH_TIME_3 1.32, 0.269, 2.49, 5.67, 11.0, 0.036, 0.119, 0.0
+#define QH_TIME_4 2.19, 0.236, 2.16, 5.67, 8.42, 0.083, 0.132, 0.718
+#define QH_TIME_5 3.49, 0.664, 0.0, 2.99, 12.0, 0.839, 0.0644, 0.219
+#define QH_TIME_6 2.76, 1.11, 0.91, 2.93, 3.54, 1.18, 0.0562, 0.429
+#define QH_TIME_7 2.72, 1.07, 0.555, 0.0, 7.05, 1.37, 0.0425, 0.291
+#define QH_TIME_8 3.17, 1.48, 0.0, 0.0, 3.81, 2.06, 0.0658, 0.351
+#define QH_TIME_9 3.18, 1.05, 1.74, 0.0, 5.92, 1.81, 0.0443, 0.261
 constexpr TileShape kTiles[] = {QH_TILE_SHAPES(QH_V)};
 #undef QH_V
+
+// The same of the ring kernel:
+//   start + max(unit turns, share load) KB + turn turns + weights nMB + out oMB
+//   + x cX + xcd dX
+// load: (tile, K slice) items per CU of the busiest XCD, which owns ceil(N tiles
+// / 8) of them with all row tiles (dma_tile); turns: items its busiest workgroup
+// takes one after the other; KB: K blocks of an item; unit, share: us per K block
+// of a workgroup alone (latency) and of its share of a full CU (throughput); cX:
+// MB of X that a CU takes in on average; dX: MB of X that reach the XCDs.
+// Rms error 3 - 4 %.  (Counting tiles over the whole chip instead booked two
+// rounds of 1345 .. 1600 x 2560 x 9216 as one: 82 us modelled, 145 measured.)
+struct RingTime {
+  int bm, bn, wpc;
+  double start, unit, share, turn, weights, out, x, xcd;
+};
+constexpr RingTime kRings[] = {{64, 64, 3, 3.18, 0.657, 0.313, 0.0, 0.0749, 0.330, 1.56, 0.0211},
+                               {64, 128, 2, 3.11, 0.826, 0.449, 0.323, 0.0676, 0.199, 5.89, 0.0199},
+                               {128, 192, 1, 3.39, 1.33, 1.21, 3.08, 0.0792, 0.033, 7.13, 0.0210}};
 
 inline long tiles_of(const QhGemmSeg* seg, int nseg, int bn) {
   long n = 0;
   for (int t = 0; t < nseg; ++t) n += (seg[t].N + bn - 1) / bn;
   return n;
+}
+inline long ceil_div(long a, long b) { return (a + b - 1) / b; }
+
+// What follows a GEMM: the finish of S K slices (part MB of partials, written and
+// read), with a lone segment fused with the residual add and the norm, or without
+// slices the add + norm launch (out MB): a lone segment is an output projection,
+// and gets the same plan (the same bits) without the add and norm.
+inline double finish_time(bool ring, int S, bool lone, double part, double out) {
+  if (S == 1) return lone ? 2.58 + 0.522 * out : 0.0;
+  return (lone ? 2.91 : 3.12) + (ring ? 0.316 : 0.466) * part + (ring ? 0.146 : 0.101) * (S - 1);
 }
 
 // The plan with the shortest modelled time.
@@ -1024,68 +1057,89 @@ inline long tiles_of(const QhGemmSeg* seg, int nseg, int bn) {
 //    tile stay in registers).  Tiles narrower than the shape's when they all
 //    run at once: the CUs then share the weight bytes evenly (2560 x 9216, 24
 //    rows: 13.9 us with 16 columns, 13.2 with 12).
-//  - Split K (caller workspace only): the partials' round trip and the
-//    finishing launch; a lone segment is an output projection, whose finish
-//    replaces the add + norm launch that would follow.
-//  - Ring kernel beside it where its model holds and the tile shapes leave
-//    CUs idle: one 64 x 64 tile per CU (1024 x 1024 x 2560: 15.4 us against
-//    17.9), one or two rounds of 64 x 128 at two workgroups per CU (400 x 8192 x
-//    2560: 27.3 against 30.4; 416 x 18432 x 2560: 53.4 against 58.7).  Every other ring plan lost (3700 x 18432 x 2560: 387
-//    against 346 us; 24 x 2560 x 9216: 48 against 12).
+//  - Split K: with a caller workspace that holds the partials.
+//  - Ring kernel beside it, all of its plans: its persistent workgroups run
+//    several per CU and overlap one tile's stores with the next one's loads, so
+//    it wins where the tile shapes leave CUs idle or K is short (640 x 2560 x
+//    9216 with K in two slices: 52.6 us against 57.4 of the best tile shape; 913 x
+//    10240 x 2560: 66 against 74; 2852 x 515 x 640: 9.2 against 10.1) and loses
+//    elsewhere (3700 x 18432 x 2560: 387 against 346; 1536 x 2560 x 9216: 123
+//    against 100; 24 x 2560 x 9216: 48 against 12).
+//  - Over 4800 shapes the plan is 0.3 % slower than the fastest one measured on
+//    average, more than 6 % slower at 1 % of them.
 //  - Other scale modes: the ring kernel's own plans (gemm_plan_ring).
 GemmPlan gemm_plan_ring(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const void* ws, size_t ws_bytes);
 
 GemmPlan gemm_plan(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const void* ws, size_t ws_bytes) {
   const int KB = K / 128;
-  long nsum = 0;
+  long nsum = 0, nodd = 0;
   bool block = KB >= 2 && KB <= 128;
   for (int t = 0; t < nseg; ++t) {
     block = block && seg[t].kb == KB;
     nsum += seg[t].N;
+    if (seg[t].N % 4 != 0 || (uintptr_t)seg[t].y % 8 != 0) nodd += seg[t].N;
   }
   if (!block) return gemm_plan_ring(M, K, seg, nseg, cus, ws, ws_bytes);
-  GemmPlan best = {-1, 64, 64, 3, 64, 1, 0};
+  const long xcd_cus = cus >= 8 ? cus / 8 : 1;
+  const double wmb = (double)nsum * K * 1e-6, xmb = 2e-6 * M * K, omb = 2e-6 * M * (double)nsum;
+  GemmPlan best = {};
   double best_t = 1e300;
-  const long r64 = (long)((M + 63) / 64) * tiles_of(seg, nseg, 64), r128 = (long)((M + 63) / 64) * tiles_of(seg, nseg, 128);
-  if (r64 <= cus) best_t = 2.8 + 0.61 * KB;
-  const double t128 = (double)((r128 + 2L * cus - 1) / (2L * cus)) * (5.39 + 1.06 * KB);
-  if (r128 > cus && r128 <= 4L * cus && t128 < best_t) {
-    best_t = t128;
-    best = {-1, 64, 128, 2, 128, 1, 0};
+// (unrolled: the shapes' numbers become constants, no divisions by them)
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(kRings) / sizeof(kRings[0])); ++i) {
+    const RingTime& c = kRings[i];
+    const long tiles_n = tiles_of(seg, nseg, c.bn), tiles_m = ceil_div(M, c.bm);
+    for (int S = 1; S <= (ws ? 8 : 1); ++S) {
+      const size_t part = (size_t)S * M * tiles_n * c.bn * sizeof(float);
+      if (S > 1 && (KB % S != 0 || KB / S < 4 || part > ws_bytes)) continue;
+      const long items = tiles_m * ceil_div(tiles_n, 8) * S;
+      const long load = ceil_div(items, xcd_cus), turns = ceil_div(items, xcd_cus * c.wpc);
+      double t = c.start + std::max(c.unit * (double)turns, c.share * (double)load) * (KB / S) + c.turn * (double)turns;
+      t += c.weights * wmb + (S == 1 ? c.out * omb : 0.0) + c.x * xmb * (double)tiles_n / cus;
+      t += c.xcd * xmb * (double)min(8L, tiles_n) + finish_time(true, S, nseg == 1, (double)part * 1e-6, omb);
+      if (t < best_t) {
+        best_t = t;
+        best = {-1, c.bm, c.bn, c.wpc, c.bn, S, (int)(tiles_n * c.bn), load};
+      }
+    }
   }
+#pragma unroll
   for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
     const TileShape& c = kTiles[i];
-    const long tiles_m = (M + c.bm - 1) / c.bm;
-    for (int S = 1; S <= 8; S *= 2) {
+    const long tiles_m = ceil_div(M, c.bm);
+    for (int S = 1; S <= (c.split && ws ? 8 : 1); S *= 2) {
       int nstep = c.bn;
       long tiles_n = tiles_of(seg, nseg, nstep);
+      const size_t part = (size_t)S * M * tiles_n * nstep * sizeof(float);
       if (S > 1) {
-        if (!c.split || !ws || KB % S != 0 || (size_t)S * M * tiles_n * nstep * sizeof(float) > ws_bytes) continue;
+        if (KB % S != 0 || part > ws_bytes) continue;
       } else if (tiles_m * tiles_n <= cus) {
         nstep = (int)min((long)c.bn, (nsum * tiles_m / cus + 3) / 4 * 4);
         nstep = nstep < 4 ? 4 : nstep;
         while (nstep < c.bn && tiles_m * tiles_of(seg, nseg, nstep) > cus) nstep += 4;
         tiles_n = tiles_of(seg, nseg, nstep);
       }
-      const long rounds = (tiles_m * tiles_n * S + cus - 1) / cus;
+      // tiles of an XCD: an eighth of them, or with 8 slices one slice of each
+      const long T = tiles_m * tiles_n, rounds = ceil_div(S == 8 ? T : ceil_div(T * S, 8), xcd_cus);
       const int units = (K / c.ku + S - 1) / S, passes = (units + c.kg - 1) / c.kg;
-      const double mb = (double)rounds * (2.0 * min(M, c.bm) + nstep) * K / S * 1e-6;
-      double t = c.a + c.b * (double)rounds * passes + c.c * (double)rounds + c.d * mb;
-      if (S > 1) t += (nseg == 1 ? 1.0 : 3.0) + (S + 0.5) * M * (double)tiles_n * nstep * 1e-6;
-      if (t < best_t * 0.99) {
+      double t = c.pass * passes + c.round + (2.0 * c.x * min(M, c.bm) + c.w * nstep) * K / S * 1e-6;
+      if (S == 1) t += c.odd * (double)nodd / (double)nsum;
+      t = c.start + (double)rounds * t + c.weights * wmb + (S == 1 ? c.out * omb : 0.0);
+      t += finish_time(false, S, nseg == 1, (double)part * 1e-6, omb);
+      if (t < best_t) {
         best_t = t;
-        best = {i, c.bm, c.bn, 1, nstep, S, (int)(tiles_n * nstep)};
+        best = {i, c.bm, c.bn, 1, nstep, S, (int)(tiles_n * nstep), rounds};
       }
     }
   }
   return best;
 }
 
-// Cycles one workgroup of the ring kernel spends per (tile, 128-wide K block)
-// unit at its occupancy (64 x 64: three workgroups per CU, 64 x 128: two,
-// 128 x 192: one), measured on MI355X at M = 512 (X fits the XCD's L2) and at
-// M = 3700 (grouped row tiles; X streams): 2.0 / 2.2 / 4.3 and 2.5 / 2.6 / 3.8
-// thousand.
+// Other scale modes: cycles one workgroup of the ring kernel spends per (tile,
+// 128-wide K block) unit at its occupancy (64 x 64: three workgroups per CU, 64 x
+// 128: two, 128 x 192: one), measured on MI355X at M = 512 (X fits the XCD's L2)
+// and at M = 3700 (grouped row tiles; X streams): 2.0 / 2.2 / 4.3 and 2.5 / 2.6 /
+// 3.8 thousand.
 struct GemmShape {
   int bm, bn, wpc;
   double cycles_small, cycles_large;
@@ -1099,7 +1153,7 @@ constexpr GemmShape kGemmShapes[] = {{64, 64, 3, 2030.0, 2460.0}, {64, 128, 2, 2
 // round trip through memory and the finishing launch (≈ 6 us).
 GemmPlan gemm_plan_ring(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const void* ws, size_t ws_bytes) {
   const int KB = K / 128;
-  GemmPlan best = {-1, 64, 64, 3, 64, 1, 0};
+  GemmPlan best = {};
   double best_t = 1e300;
   for (const GemmShape& c : kGemmShapes) {
     const long tiles_n = tiles_of(seg, nseg, c.bn);
@@ -1115,7 +1169,7 @@ GemmPlan gemm_plan_ring(int M, int K, const QhGemmSeg* seg, int nseg, int cus, c
       if (S > 1) t += (double)S * M * tiles_n * c.bn * 4.0 * 2.0 / 2048.0 + 13000.0;
       if (t < best_t * 0.98) {
         best_t = t;
-        best = {-1, c.bm, c.bn, c.wpc, c.bn, S, (int)(tiles_n * c.bn)};
+        best = {-1, c.bm, c.bn, c.wpc, c.bn, S, (int)(tiles_n * c.bn), ceil_div(items, cus >= 8 ? cus / 8 : 1)};
       }
     }
   }
@@ -1162,6 +1216,16 @@ size_t qh_gemm_workspace_bytes(int M, int K) {
   return kSplitPartBytes;
 }
 
+namespace {
+int device_cus() {
+  int cus = 256, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    cus = 256;
+  return cus;
+}
+}  // namespace
+
 int qh_launch_gemm_e4m3_group_ws(const void* x, int M, int K, const QhGemmSeg* seg, int nseg,
                                  bool scale_bf16, void* ws, size_t ws_bytes, hipStream_t st) {
   if (K <= 0 || K % 128 != 0 || M <= 0) {
@@ -1186,10 +1250,7 @@ int qh_launch_gemm_e4m3_group_ws(const void* x, int M, int K, const QhGemmSeg* s
   }
   const uint16_t* xa = (const uint16_t*)x;
   const long mt = (M + kBM - 1) / kBM;
-  int cus = 256, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    cus = 256;
+  const int cus = device_cus();
   // 64x64 tiles: with the activation used as is, wider tiles only cut
   // occupancy or (weights loaded straight into operand registers) the load
   // path's coalescing.
@@ -1214,10 +1275,24 @@ int qh_launch_gemm_e4m3_group_ws(const void* x, int M, int K, const QhGemmSeg* s
   return 0;
 }
 
+int qh_gemm_plan_of(int M, int K, const int* N, int nseg, int kb, int cus, size_t ws_bytes, int* out) {
+  if (M <= 0 || K <= 0 || K % 128 != 0 || nseg < 1 || nseg > 4 || cus <= 0 || !N || !out) return -1;
+  QhGemmSeg seg[4] = {};
+  for (int t = 0; t < nseg; ++t) {
+    if (N[t] <= 0) return -1;
+    seg[t].N = N[t];
+    seg[t].kb = kb;
+  }
+  const GemmPlan pl = gemm_plan(M, K, seg, nseg, cus, ws_bytes ? (const void*)seg : nullptr, ws_bytes);
+  const int v[] = {pl.tile, pl.bm, pl.bn, pl.wpc, pl.nstep, pl.S, (int)pl.load};
+  for (int i = 0; i < 7; ++i) out[i] = v[i];
+  return 0;
+}
+
 // Output projection + residual + norm (the batch prefill's o_proj / out_proj /
 // down): o = bf16(x W^T), h = bf16(h + o), hn = (1+w) RMSNorm(h) (none when
-// norm_w is null).  When the GEMM splits K through the ring kernel and the
-// rows fit its vector kernel, one row-wise kernel finishes the split, the add
+// norm_w is null).  When the GEMM splits K (tile or ring kernel) and the rows
+// fit its vector kernel, one row-wise kernel finishes the split, the add
 // and the norm (o is not written); otherwise o is written and the fused
 // add + norm kernel follows.
 int qh_launch_gemm_e4m3_add_rmsnorm(const void* x, const void* w, const void* s, void* o, int M, int N, int K,
@@ -1227,10 +1302,7 @@ int qh_launch_gemm_e4m3_add_rmsnorm(const void* x, const void* w, const void* s,
   if (M > 0 && N > 0 && K > 0 && K % 128 == 0 && ws && x && (uintptr_t)x % 16 == 0 && w && s &&
       (uintptr_t)w % 16 == 0 && (uintptr_t)s % 4 == 0 && gemm_dma_fits(K) && N % 8 == 0 && N <= 8192 &&
       al16(h) && al16(hn) && al16(norm_w)) {
-    int cus = 256, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      cus = 256;
+    const int cus = device_cus();
     const QhGemmSeg seg = {w, s, o, N, kb};
     const GemmPlan pl = gemm_plan(M, K, &seg, 1, cus, ws, ws_bytes);
     if (pl.S > 1) {
