@@ -956,10 +956,9 @@ __global__ __launch_bounds__(256) void gdn_front_kernel(QhGdnPrepParams p) {
   for (int k = 0; k < T; ++k) {
     const int m = m0 + k;
     u32x4 out;
-    float ss = 0.0f;
+    float ss = 0.0f, r[8];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      float r2[2];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int e = 4 * (2 * q + h);  // tap j of channel 2 q + h is element e + j of the 32
@@ -972,9 +971,13 @@ __global__ __launch_bounds__(256) void gdn_front_kernel(QhGdnPrepParams p) {
         acc = fmaf(wt(2), xv(1), acc);
         acc = fmaf(wt(1), xv(2), acc);
         acc = fmaf(wt(0), xv(3), acc);
-        r2[h] = qh_silu_bf(rbf(acc));
+        r[2 * q + h] = rbf(acc);
       }
-      out[q] = pack_bf2(r2[0], r2[1]);
+    }
+    qh_silu_bf(r);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      out[q] = pack_bf2(r[2 * q], r[2 * q + 1]);
       const float y0 = bf_lo(out[q]), y1 = bf_hi(out[q]);
       ss += rbf(y0 * y0) + rbf(y1 * y1);
     }
@@ -1123,11 +1126,18 @@ __global__ __launch_bounds__(256) void gdn_gated_norm_wave_kernel(QhGdnScanParam
     ss = fmaf(bf_hi(cv[q]), bf_hi(cv[q]), ss);
   }
   const float rs = rsqrtf(column_sum<16>(ss) / 128.0f + p.eps);
+  float z[8];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    z[2 * q] = bf_lo(zv[q]);
+    z[2 * q + 1] = bf_hi(zv[q]);
+  }
+  qh_silu_bf(z);
   u32x4 y;
 #pragma unroll
   for (int q = 0; q < 4; ++q)
-    y[q] = pack_bf2(rbf(rbf(bf_lo(cv[q]) * rs) * bf_lo(wv[q])) * rbf(qh_silu_bf(bf_lo(zv[q]))),
-                    rbf(rbf(bf_hi(cv[q]) * rs) * bf_hi(wv[q])) * rbf(qh_silu_bf(bf_hi(zv[q]))));
+    y[q] = pack_bf2(rbf(rbf(bf_lo(cv[q]) * rs) * bf_lo(wv[q])) * rbf(z[2 * q]),
+                    rbf(rbf(bf_hi(cv[q]) * rs) * bf_hi(wv[q])) * rbf(z[2 * q + 1]));
   *(u32x4*)(p.out + o) = y;
 }
 __global__ __launch_bounds__(128) void gdn_gated_norm_kernel(QhGdnScanParams p) {

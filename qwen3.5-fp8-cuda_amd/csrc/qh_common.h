@@ -209,23 +209,35 @@ __device__ __forceinline__ void reset_counter(unsigned* counter) {
 // flips and a per-step bias against the reference's fp32 torch ops.
 __device__ __forceinline__ float qh_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float qh_silu(float x) { return x / (1.0f + expf(-x)); }
-// SiLU whose argument is a bf16 value and whose result is rounded to bf16, for
-// loops that its arithmetic bounds: e^-x as 2^t with the rounding of
-// t = -x log2(e) corrected to first order, and one Newton step on the hardware
-// reciprocal's quotient, 12 instructions in place of expf's and the IEEE
-// division's 25.  Over all finite bf16 arguments it rounds to the bf16 value
-// that 64-bit arithmetic gives at least as often as fp32 arithmetic with expf
-// does (test_conv_silu_every_argument).  Above 88 it is x (as in fp32, infinity
-// included), below -88 zero or a denormal; NaN stays NaN.
-__device__ __forceinline__ float qh_silu_bf(float x) {
-  const float a = fminf(-x, 88.0f);
-  const float t = a * 1.44269502f;                                // log2(e), high part
-  const float c = fmaf(a, 1.92596299e-8f, fmaf(a, 1.44269502f, -t));  // low part and t's rounding
-  const float e = __builtin_amdgcn_exp2f(t);
-  const float d = 1.0f + fmaf(e, c * 0.693147182f, e);
-  const float q = x * __builtin_amdgcn_rcpf(d);
-  const float y = fmaf(fmaf(-q, d, x), __builtin_amdgcn_rcpf(d), q);
-  return x > 88.0f ? x : y;
+// SiLU of N bf16 values, in place, whose results are rounded to bf16, for loops
+// that its arithmetic bounds: e^-x as 2^t with the rounding of t = -x log2(e)
+// corrected to first order, and one Newton step on the hardware reciprocal's
+// quotient, 11 instructions in place of expf's and the IEEE division's 25.  Over
+// all finite bf16 arguments it rounds to the bf16 value that 64-bit arithmetic
+// gives at least as often as fp32 arithmetic with expf does
+// (test_conv_silu_every_argument).  Above 87 in magnitude, where the reciprocal
+// would be denormal (the hardware flushes it) or a step overflows, a value takes
+// the fp32 form, infinities included: one branch for all N.  NaN stays NaN.
+template <int N>
+__device__ __forceinline__ void qh_silu_bf(float (&x)[N]) {
+  float big = 0.0f, y[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    big = fmaxf(big, fabsf(x[i]));
+    const float t = x[i] * -1.44269502f;  // -log2(e), high part
+    // its low part and t's rounding
+    const float c = fmaf(x[i], -1.92596299e-8f, fmaf(x[i], -1.44269502f, -t));
+    const float e = __builtin_amdgcn_exp2f(t);
+    const float d = 1.0f + fmaf(e, c * 0.693147182f, e);
+    const float r = __builtin_amdgcn_rcpf(d), q = x[i] * r;
+    y[i] = fmaf(fmaf(-q, d, x[i]), r, q);
+  }
+  if (big > 87.0f) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) y[i] = fabsf(x[i]) > 87.0f ? qh_silu(x[i]) : y[i];
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = y[i];
 }
 // Sigmoid of a bf16 value whose result is rounded to bf16, by the same steps:
 // e^-x corrected to first order, one Newton step on the hardware reciprocal.

@@ -75,6 +75,10 @@ def test_conv_silu_every_argument(M):
     normal = exact.abs() > 1e-36
     assert int((y != exact)[normal].sum()) <= int((f32 != exact)[normal].sum())
     assert ((y - exact).abs() <= 2.0 ** -7 * exact.abs() + 1e-36).all()
+    # the lower end, where e^-x nears the largest fp32 number: normal results down to -88.5, zero below as
+    # in fp32 (1 + e^-x is infinite there)
+    low = x.float() <= -87.0
+    assert int((f32[low] != 0).sum()) >= 4 and ((y - f32).abs() <= 2.0 ** -7 * f32.abs())[low].all()
     x = torch.zeros(M, C, dtype=torch.bfloat16)
     x[-1, :3] = torch.tensor([float("inf"), -float("inf"), float("nan")])
     y = front(x, torch.zeros(C, 4, dtype=torch.bfloat16), w, z, z, torch.zeros(1), torch.zeros(1), 1, 1, 0)[0].float()
