@@ -1052,6 +1052,17 @@ inline double finish_time(bool ring, int S, bool lone, double part, double out) 
   return (lone ? 2.91 : 3.12) + (ring ? 0.316 : 0.466) * part + (ring ? 0.146 : 0.101) * (S - 1);
 }
 
+// X as the kernel before has left it, which the shapes were not fitted with (they
+// read X out of the L2s): every XCD of the ring kernel reads all of X; of the tile
+// kernel with 8 slices an eighth, else the rows of its tiles, in groups of 4 row
+// tiles.  Fitted to the MLP and the output projections of 52 row counts in their
+// place between other kernels (128 x 2560 x 9216: the ring with 6 slices and the 64
+// x 160 tiles with 8 take 19.5 us alone, in place the tiles are 1.4 us faster).
+inline double fresh_x_ring(double xmb) { return 0.24 * xmb; }
+inline double fresh_x_tile(double xmb, int S, long tiles_m) {
+  return 0.08 * xmb * (S == 8 ? 1.0 : std::max(1.0, std::min(8.0, 32.0 / (double)tiles_m)));
+}
+
 // The plan with the shortest modelled time.
 //  - Tile kernel: 128 x 128 block scales, up to 128 K blocks (the scales of a
 //    tile stay in registers).  Tiles narrower than the shape's when they all
@@ -1096,7 +1107,8 @@ GemmPlan gemm_plan(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const 
       const long load = ceil_div(items, xcd_cus), turns = ceil_div(items, xcd_cus * c.wpc);
       double t = c.start + std::max(c.unit * (double)turns, c.share * (double)load) * (KB / S) + c.turn * (double)turns;
       t += c.weights * wmb + (S == 1 ? c.out * omb : 0.0) + c.x * xmb * (double)tiles_n / cus;
-      t += c.xcd * xmb * (double)min(8L, tiles_n) + finish_time(true, S, nseg == 1, (double)part * 1e-6, omb);
+      t += c.xcd * xmb * (double)min(8L, tiles_n) + fresh_x_ring(xmb);
+      t += finish_time(true, S, nseg == 1, (double)part * 1e-6, omb);
       if (t < best_t) {
         best_t = t;
         best = {-1, c.bm, c.bn, c.wpc, c.bn, S, (int)(tiles_n * c.bn), load};
@@ -1125,6 +1137,7 @@ GemmPlan gemm_plan(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const 
       double t = c.pass * passes + c.round + (2.0 * c.x * min(M, c.bm) + c.w * nstep) * K / S * 1e-6;
       if (S == 1) t += c.odd * (double)nodd / (double)nsum;
       t = c.start + (double)rounds * t + c.weights * wmb + (S == 1 ? c.out * omb : 0.0);
+      t += fresh_x_tile(xmb, S, tiles_m);
       t += finish_time(false, S, nseg == 1, (double)part * 1e-6, omb);
       if (t < best_t) {
         best_t = t;
