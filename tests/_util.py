@@ -1,4 +1,6 @@
 """Shared helpers for the parity tests."""
+import ctypes
+
 import torch
 
 from oracle import qwen35_oracle as orc
@@ -44,3 +46,22 @@ def assert_close(got, ref, rtol=1e-2, atol_frac=1e-4, min_cos=0.99999, what=""):
 
 def quant(g, n, k, std=0.02):
     return orc.quantize_block_fp8(randn(g, n, k, std=std))
+
+
+def gemm_plan(M, K, N, ws=None, kb=None, cus=256):
+    """qh_gemm_plan by field names; ws None: a workspace of the full size."""
+    from qwen35_amd import abi
+    lib, out = abi.load(), (ctypes.c_int * 7)()
+    if ws is None:
+        ws = int(lib.qh_gemm_workspace_size(M, K))
+    abi.check(lib.qh_gemm_plan(M, K, len(N), ctypes.cast((ctypes.c_int * len(N))(*N), ctypes.c_void_p),
+                               K // 128 if kb is None else kb, cus, ws, ctypes.cast(out, ctypes.c_void_p)), "plan")
+    return dict(zip(("tile", "bm", "bn", "wpc", "nstep", "S", "load"), out))
+
+
+def gemm_shape(M, K, N, ws=None, cus=256):
+    """The shape a product runs on, "t3" (tile kernel) or "r128" (ring kernel, columns of its tile), with
+    its K slices where there are several: "t3/4"."""
+    p = gemm_plan(M, K, N, ws, cus=cus)
+    name = f"t{p['tile']}" if p["tile"] >= 0 else f"r{p['bn']}"
+    return name if p["S"] == 1 else f"{name}/{p['S']}"

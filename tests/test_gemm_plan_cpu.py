@@ -6,19 +6,11 @@ import pytest
 
 from qwen35_amd import abi
 
+from _util import gemm_plan as plan
+
 CUS = 256
 PROJ = {"in_proj": (2560, (8192, 4096, 32, 32)), "qkv": (2560, (8192, 1024, 1024)),
         "o": (4096, (2560,)), "gate_up": (2560, (9216, 9216)), "down": (9216, (2560,))}
-
-
-def plan(M, K, N, ws=None, kb=None, cus=CUS):
-    lib, out = abi.load(), (ctypes.c_int * 7)()
-    if ws is None:
-        ws = int(lib.qh_gemm_workspace_size(M, K))
-    abi.check(lib.qh_gemm_plan(M, K, len(N), ctypes.cast((ctypes.c_int * len(N))(*N), ctypes.c_void_p),
-                               K // 128 if kb is None else kb, cus, ws,
-                               ctypes.cast(out, ctypes.c_void_p)), "plan")
-    return dict(zip(("tile", "bm", "bn", "wpc", "nstep", "S", "load"), out))
 
 
 def busiest_xcd(p, M, N, cus=CUS):
