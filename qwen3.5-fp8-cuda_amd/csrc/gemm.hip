@@ -1019,22 +1019,23 @@ constexpr TileShape kTiles[] = {QH_TILE_SHAPES(QH_V)};
 #undef QH_V
 
 // The same of the ring kernel:
-//   start + max(unit turns, share load) KB + turn turns + weights nMB + out oMB
-//   + x cX + xcd dX
+//   start + (max(unit turns, share load) + full) KB + turn turns + weights nMB
+//   + out oMB + x cX + xcd dX
 // load: (tile, K slice) items per CU of the busiest XCD, which owns ceil(N tiles
 // / 8) of them with all row tiles (dma_tile); turns: items its busiest workgroup
 // takes one after the other; KB: K blocks of an item; unit, share: us per K block
-// of a workgroup alone (latency) and of its share of a full CU (throughput); cX:
-// MB of X that a CU takes in on average; dX: MB of X that reach the XCDs.
-// Rms error 3 - 4 %.  (Counting tiles over the whole chip instead booked two
-// rounds of 1345 .. 1600 x 2560 x 9216 as one: 82 us modelled, 145 measured.)
+// of a workgroup alone (latency) and of its share of a full CU (throughput); full:
+// more of them when all of a CU's workgroups have an item in the last turn; cX: MB
+// of X that a CU takes in on average; dX: MB of X that reach the XCDs.  Rms error
+// 3 - 4 %.  (Counting tiles over the whole chip instead booked two rounds of
+// 1345 .. 1600 x 2560 x 9216 as one: 82 us modelled, 145 measured.)
 struct RingTime {
   int bm, bn, wpc;
-  double start, unit, share, turn, weights, out, x, xcd;
+  double start, unit, share, full, turn, weights, out, x, xcd;
 };
-constexpr RingTime kRings[] = {{64, 64, 3, 3.18, 0.657, 0.313, 0.0, 0.0749, 0.330, 1.56, 0.0211},
-                               {64, 128, 2, 3.11, 0.826, 0.449, 0.323, 0.0676, 0.199, 5.89, 0.0199},
-                               {128, 192, 1, 3.39, 1.33, 1.21, 3.08, 0.0792, 0.033, 7.13, 0.0210}};
+constexpr RingTime kRings[] = {{64, 64, 3, 2.68, 0.652, 0.289, 0.115, 0.50, 0.0697, 0.284, 2.57, 0.0060},
+                               {64, 128, 2, 3.14, 0.834, 0.454, 0.0, 0.326, 0.0683, 0.201, 5.95, 0.0201},
+                               {128, 192, 1, 3.39, 1.33, 1.21, 0.0, 3.08, 0.0792, 0.033, 7.13, 0.0210}};
 
 inline long tiles_of(const QhGemmSeg* seg, int nseg, int bn) {
   long n = 0;
@@ -1076,8 +1077,8 @@ inline double fresh_x_tile(double xmb, int S, long tiles_m) {
 //    10240 x 2560: 66 against 74; 2852 x 515 x 640: 9.2 against 10.1) and loses
 //    elsewhere (3700 x 18432 x 2560: 387 against 346; 1536 x 2560 x 9216: 123
 //    against 100; 24 x 2560 x 9216: 48 against 12).
-//  - Over 4800 shapes the plan is 0.3 % slower than the fastest one measured on
-//    average, more than 6 % slower at 1 % of them.
+//  - Over 4800 shapes the plan is 0.35 % slower than the fastest one measured on
+//    average, more than 7 % slower at 1 % of them; in place 0.4 %, at most 2.3 %.
 //  - Other scale modes: the ring kernel's own plans (gemm_plan_ring).
 GemmPlan gemm_plan_ring(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const void* ws, size_t ws_bytes);
 
@@ -1105,7 +1106,8 @@ GemmPlan gemm_plan(int M, int K, const QhGemmSeg* seg, int nseg, int cus, const 
       if (S > 1 && (KB % S != 0 || KB / S < 4 || part > ws_bytes)) continue;
       const long items = tiles_m * ceil_div(tiles_n, 8) * S;
       const long load = ceil_div(items, xcd_cus), turns = ceil_div(items, xcd_cus * c.wpc);
-      double t = c.start + std::max(c.unit * (double)turns, c.share * (double)load) * (KB / S) + c.turn * (double)turns;
+      double t = std::max(c.unit * (double)turns, c.share * (double)load) + (load == turns * c.wpc ? c.full : 0.0);
+      t = c.start + t * (KB / S) + c.turn * (double)turns;
       t += c.weights * wmb + (S == 1 ? c.out * omb : 0.0) + c.x * xmb * (double)tiles_n / cus;
       t += c.xcd * xmb * (double)min(8L, tiles_n) + fresh_x_ring(xmb);
       t += finish_time(true, S, nseg == 1, (double)part * 1e-6, omb);
