@@ -87,7 +87,7 @@ __device__ __forceinline__ f4 zero4() { return f4{0.0f, 0.0f, 0.0f, 0.0f}; }
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // ---- prep: grid (chunks, Hv), 256 threads -----------------------------------
-// Two workgroups per CU (76 KB of LDS; with K, Q, T' and both dim-major tiles
+// Two workgroups per CU (71 KB of LDS; with K, Q, T' and both dim-major tiles
 // in LDS it was one, and 3700 tokens took 115 us).
 __global__ __launch_bounds__(256, 2) void gdn_chunk_prep_kernel(QhGdnScanParams p, float* ws, int nch) {
   __shared__ __align__(16) uint16_t sKV[DV * TS];  // K token-major (stride RS), then V dim-major (stride TS)

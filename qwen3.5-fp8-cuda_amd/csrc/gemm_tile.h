@@ -31,9 +31,10 @@
 //
 // LDS rows are unpadded (direct-to-LDS loads fill whole 1 KB runs) and
 // XOR-swizzled by row in 16-byte slots.  A 16-byte read serves lanes 0-3,
-// 12-15, 20-23 and 24-27 of a half wave together, then the others; the
-// swizzles put each such group in different banks (no conflicts by PMC; with
-// slot c ^ (r / 4) for 64-byte rows half of the cycles were conflicts).
+// 12-15, 20-23 and 24-27 of a half wave together, then the others; with
+// 128-wide units the swizzles put each such group in different banks (counted:
+// no conflict cycles), with 64-wide ones 38 % of the LDS cycles still are
+// conflicts (half of them with slot c ^ (r / 4) for 64-byte rows).
 // LDS reads are inline asm, which the compiler does not count against the
 // loads in flight; every read is waited for, by count and tied to its
 // registers, before use.

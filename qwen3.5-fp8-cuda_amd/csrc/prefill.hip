@@ -343,6 +343,11 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(QhAttnPrefillParams p
 // p <= e^kFaSlack and O / l is unchanged up to fp32 rounding; most tiles skip
 // the 128-accumulator rescale.
 //
+// A block of 32 queries shares its tiles' P . V products, the masked positions
+// (p = 0) included, as a dense softmax . V does: a V row that is not finite
+// reaches up to 31 tokens before its own, where the per-token kernel keeps to the
+// positions a token sees.
+//
 // Precision as the reference's fp32 q . k, softmax and P . v: q (fp32) and P
 // (fp32) enter as hi + lo bf16 pairs (hi = bf16(x), lo = bf16(x - hi), about
 // 16 mantissa bits), each pair two matrix-core products that are exact in
@@ -662,6 +667,8 @@ __device__ __forceinline__ void fa_tiles(FaWave<NL>& w, int nt, int tmask, AT at
   }
 }
 
+// (132 bytes of scratch per lane: query operands that the branch for low parts in
+// every dimension saves outside its tile loop; the other branch touches none.)
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void attn_prefill_mfma_kernel(
     QhAttnPrefillParams p) {
 #ifdef __HIP_DEVICE_COMPILE__

@@ -37,8 +37,10 @@ def rope_tables(max_pos, rotary_dim, theta, device="cpu"):
 
 # Prompts of at least this many tokens run the GatedDeltaNet layers in the
 # chunked (WY) form on the matrix cores (qh_gdn_chunk); shorter ones use the
-# recurrent scan.  At the 4B shape the chunked form measured 38 us against
-# 50 us per layer at 128 tokens and 32 us against 31 us at 64.
+# recurrent scan.  The line was drawn where the chunk kernels of then (32 us at 64
+# tokens) passed the scan; at the 4B shape the two now take, with the gated norm,
+# 20.8 and 48.1 us per layer at 128 tokens, 20.2 and 39.2 at 96, 18.0 and 30.5 at
+# 64, 16.7 and 21.3 at 32.
 GDN_CHUNK_MIN_TOKENS = 96
 
 
