@@ -1230,13 +1230,18 @@ int qh_launch_attn_prefill(const QhAttnPrefillParams& p, hipStream_t st) {
   }
   if (p.M <= 0) return 0;
   // D = 256 with 4 query heads per KV head, 16-byte aligned rows and a last
-  // token that sees at least 256 positions: the matrix-core kernel (one
-  // workgroup per 32 tokens); other launches the per-token one.  A workgroup of
-  // the first takes 18 us and 2.0 us per 64 positions, one of the second 3 us
-  // and 2.6 us per 32 positions.  Measured per layer at 4 KV heads, per-token
-  // vs matrix-core: 128 tokens 14 vs 22 us, 224 tokens 28.5 vs 26 us, 128
-  // tokens after 1000 118 vs 54 us, 128 after 3000 304 vs 117 us.
-  if (p.past + p.M >= 256 && p.D == 256 && p.Hq == 4 * p.Hkv && (uintptr_t)p.q % 16 == 0 && (uintptr_t)p.gate % 8 == 0 &&
+  // token that sees enough positions: the matrix-core kernel (one workgroup per
+  // 32 tokens); other launches the per-token one.  A workgroup of the first takes
+  // 18 us (less with few tokens) and 2.0 us per 64 positions, one of the second
+  // 3 us and 2.4 us per 32 positions.  The line is at 256 positions, and where the
+  // per-token workgroups have a CU each and the first kernel's blocks more than a
+  // few tokens it rises with these to 368.  Measured per layer at 4 KV heads,
+  // per-token vs matrix-core: 5 tokens that see 256 23.2 vs 22.6 us; 16 tokens,
+  // 256 23.4 vs 26.0, 320 28.4 vs 28.2; 32 tokens, 256 23.7 vs 29.0, 320 28.9 vs
+  // 31.9, 384 33.9 vs 34.8, 512 43.8 vs 39.0; 64 tokens, 256 24.6 vs 30.7, 512
+  // 45.2 vs 39.8; 128 tokens, 256 28.8 vs 28.6, 1024 102 vs 57.
+  const int few = p.M <= 64 && p.Hkv * p.M <= 256 ? std::min(std::max(6 * (p.M - 6), 0), 112) : 0;
+  if (p.past + p.M >= 256 + few && p.D == 256 && p.Hq == 4 * p.Hkv && (uintptr_t)p.q % 16 == 0 && (uintptr_t)p.gate % 8 == 0 &&
       p.gate_mstride % 4 == 0 && p.gate_hstride % 4 == 0 && (uintptr_t)p.k_cache % 16 == 0 &&
       (uintptr_t)p.v_cache % 16 == 0 && (uintptr_t)p.out % 8 == 0) {
     hipLaunchKernelGGL(attn_prefill_mfma_kernel, dim3(p.Hkv, (p.M + 31) / 32), dim3(256), (size_t)kFaLds, st, p);

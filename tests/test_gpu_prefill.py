@@ -23,8 +23,8 @@ def cu(t):
 
 
 # (tokens, past): positions 0 .. past-1 are cached by an earlier prep call,
-# positions past .. tokens-1 are the prefill.  From 256 positions on the
-# matrix-core kernel runs (300: a ragged last 32-token block; 330 - 70 =
+# positions past .. tokens-1 are the prefill.  From 256 positions on (more for
+# 7 to 64 tokens) the matrix-core kernel runs (300: a ragged last 32-token block; 330 - 70 =
 # 260 after a cached prefix), below that the per-token kernel.
 # The last two cases take the per-token kernel with two query heads per wave
 # (8 per KV head, head dim 128) and with an idle wave (3 per KV head).
@@ -112,7 +112,8 @@ def test_attention_prep_vector_rows(M, past, rot, norm):
 # 2^-8 relative each (8 significant bits: half an ulp of a value just above a
 # power of two), and 2^-16 per operand from the split q and p.
 @pytest.mark.parametrize("M,past,Hkv,split_all", [(1, 255, 2, False), (5, 251, 1, True), (33, 256, 2, False),
-                                                  (257, 0, 1, True), (65, 700, 2, False), (200, 1848, 1, False)])
+                                                  (33, 352, 2, False), (257, 0, 1, True), (65, 700, 2, False),
+                                                  (200, 1848, 1, False)])
 def test_attention_prefill_matrix_cores(M, past, Hkv, split_all):
     g = gen(5 + M)
     D, Hq, max_seq = 256, 4 * Hkv, 2048
@@ -136,6 +137,28 @@ def test_attention_prefill_matrix_cores(M, past, Hkv, split_all):
         ref[:, h] = torch.softmax(sc.masked_fill(mask, -math.inf), -1) @ vc[h // 4, :end].double()
     ref = (ref * torch.sigmoid(gate.double())).reshape(M, -1)
     assert_close(out, ref.float(), rtol=3 * 2 ** -8 + 2 ** -12, atol_frac=2 ** -14, what="matrix-core attention")
+
+
+# Which kernel a call takes, on both sides of the line: it rises from 256 visible
+# positions with the tokens, from 7 to 64 of them while a KV head's tokens have a CU
+# each, up to 368.  The routes differ in what a NaN in V at the last position reaches:
+# the matrix-core kernel's whole block of 32 tokens, or the last token alone.
+@pytest.mark.parametrize("M,vis,Hkv,blocks", [(6, 255, 4, False), (6, 256, 4, True), (20, 339, 4, False),
+                                              (20, 340, 4, True), (40, 367, 4, False), (40, 368, 4, True),
+                                              (64, 367, 4, False), (64, 367, 5, True), (66, 256, 1, True),
+                                              (66, 255, 1, False)])
+def test_attention_prefill_route(M, vis, Hkv, blocks):
+    g = gen(17)
+    D, Hq, past = 256, 4 * Hkv, vis - M
+    q, gate = cu(randn(g, M, Hq, D)), cu(bf(randn(g, M, Hq, D)))
+    kc, vc = cu(bf(randn(g, Hkv, vis, D))), cu(bf(randn(g, Hkv, vis, D)))
+    vc[:, vis - 1] = float("nan")
+    out = torch.empty(M, Hq * D, dtype=torch.bfloat16, device=DEV)
+    abi.check(abi.load().qh_attn_prefill(abi.ptr(q), abi.ptr(gate), Hq * D, D, abi.ptr(kc), abi.ptr(vc), abi.ptr(out),
+                                         M, Hq, Hkv, D, past, vis, abi.stream_handle()))
+    torch.cuda.synchronize()
+    assert out[-1].isnan().all()
+    assert out[-2].isnan().all() if blocks else out[:-1].isfinite().all()
 
 
 # Every bf16 gate: with zero keys and values of one, attention is one and the
