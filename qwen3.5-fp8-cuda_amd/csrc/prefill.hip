@@ -91,8 +91,8 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(QhAttnPrepParams p) {
 // The same for D = 256 and rows aligned to what a lane moves (16 bytes of fp32, 8
 // of bf16): NR rows per wave, all of their loads ahead of the arithmetic.  Memory
 // bounds it: with 2-byte accesses and one row per wave, 3700 tokens (135 MB) took
-// 28.2 us, with this 23.0; short prompts take NR = 1, whose waves are their
-// parallelism.
+// 28.2 us, with this 23.0 (inputs still cached); prompts whose bytes are not yet
+// the bound take NR = 1, whose waves are their parallelism.
 template <int NR>
 __global__ __launch_bounds__(256) void attn_prep256_kernel(QhAttnPrepParams p) {
   constexpr int D = 256;
@@ -1207,7 +1207,10 @@ int qh_launch_attn_prep(const QhAttnPrepParams& p, hipStream_t st) {
   for (const void* q : al8) aligned = aligned && (uintptr_t)q % 8 == 0;
   // (rows stay below 2^31 - 2^10: the index of a wave's row is an int)
   if (p.D == 256 && aligned && rows < 0x7FFFFC00L) {
-    if (rows >= 8192)
+    // four rows per wave once memory bounds it: 20 rows a token, 1024 tokens 11.5 us
+    // against 10.9 with one, 2048 20.8 against 20.9, 2560 24.3 against 26.1, 3700
+    // 32.8 against 36.8
+    if (rows >= 40960)
       hipLaunchKernelGGL(attn_prep256_kernel<4>, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, st, p);
     else
       hipLaunchKernelGGL(attn_prep256_kernel<1>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, p);

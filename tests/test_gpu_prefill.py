@@ -78,14 +78,15 @@ def test_attention_prefill(M, past, Hq, Hkv, D):
     assert_close(out, ref[past:], atol_frac=1e-3, what="prefill attention")
 
 
-# The vector head-norm kernel (four rows per wave from 8192 rows on: 823 tokens x
+# The vector head-norm kernel (four rows per wave from 40960 rows on: 4097 tokens x
 # 10 rows, no multiple of its 16 rows a workgroup; else one) against the general
 # one, which a q output 4 bytes off takes: the same arithmetic, the same bits.
 @pytest.mark.parametrize("M,past,rot,norm", [(823, 0, 64, True), (823, 9, 256, True), (7, 3, 64, True),
+                                             (4095, 0, 64, True), (4097, 9, 256, True), (4097, 0, 0, False),
                                              (1, 0, 8, False), (823, 0, 0, False)])
 def test_attention_prep_vector_rows(M, past, rot, norm):
     g = gen(31 + M + rot)
-    Hq, Hkv, D, max_seq = 8, 2, 256, 840
+    Hq, Hkv, D, max_seq = 8, 2, 256, max(840, M + past)
     q, k, v = cu(bf(randn(g, M, Hq, 2 * D))), cu(bf(randn(g, M, Hkv, D))), cu(bf(randn(g, M, Hkv, D)))
     qn, kn = cu(randn(g, D, std=0.1)), cu(randn(g, D, std=0.1))
     cos, sin = (cu(t) for t in orc.rope_tables(max_seq, max(rot, 2), 1e7))
