@@ -899,23 +899,24 @@ __global__ __launch_bounds__(256) void gdn_norm_gates_kernel(QhGdnPrepParams p) 
 }
 
 // ---- conv, l2norm and gates in one pass -------------------------------------
-// One thread per 8 channels (16-byte accesses) and T consecutive tokens, whose
-// inputs slide through registers: T + 3 loads for T outputs where a thread per
-// token takes 4 T.  16 lanes hold the 128 channels of a head, so a q or k
-// head's sum of squares is a 16-lane DPP sum and its normalised row is stored
-// from the same registers.  Blocks of 4 waves, 16 T tokens; blockIdx.y < C / 128:
-// that row of 128 channels, C / 128: the gates.  The conv ring (window positions
-// before the prompt) is read by the threads of token 0's wave only, and they
-// store its new contents after their own outputs, which depend on their reads.
-// Bound by the SiLU's arithmetic from a few hundred tokens (3700 tokens: 47 us,
+// One thread per token and 8 channels (16-byte accesses).  16 lanes hold the 128
+// channels of a head, so a q or k head's sum of squares is a 16-lane DPP sum and
+// its normalised row is stored from the same registers.  Blocks of 4 waves, 16
+// tokens; blockIdx.y < C / 128: that row of 128 channels, C / 128: the gates.  The
+// conv ring (window positions before the prompt) is read by the threads of token
+// 0's wave only, and they store its new contents after their own outputs, which
+// depend on their reads.
+// Bound by the SiLU's arithmetic from a few hundred tokens (3700 tokens: 42 us,
 // 60 + 34 as a conv and a norm kernel with expf and IEEE divisions; the bytes
-// alone 35), by one round trip below (128 tokens: 4.9 us, 5.4 + 3.8).
-template <int T>
+// alone 35), by one round trip below (128 tokens: 4.9 us, 5.4 + 3.8).  8 tokens per
+// thread, whose inputs slide through registers (11 loads instead of 32), leave too
+// few waves: 17.6 us for 9.9 at 512 tokens, 33.8 for 27.7 at 2048, 48.4 for 41.9 at
+// 3700; the three earlier rows come from the caches.
 __global__ __launch_bounds__(256) void gdn_front_kernel(QhGdnPrepParams p) {
   const int wv = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int rows = p.C >> 7;
-  if ((int)blockIdx.y == rows) {  // gates of the block's 16 T tokens
-    const int m0 = (int)blockIdx.x * 16 * T, n = min(16 * T, p.M - m0) * p.Hv;
+  if ((int)blockIdx.y == rows) {  // gates of the block's 16 tokens
+    const int m0 = (int)blockIdx.x * 16, n = min(16, p.M - m0) * p.Hv;
     for (int i = threadIdx.x; i < n; i += 256) {
       const int h = i % p.Hv;
       const size_t at = (size_t)m0 * p.Hv + i;
@@ -925,14 +926,14 @@ __global__ __launch_bounds__(256) void gdn_front_kernel(QhGdnPrepParams p) {
     }
     return;
   }
-  const int m0 = (wv * 4 + (lane >> 4)) * T, c0 = (int)blockIdx.y * 128 + (lane & 15) * 8;
+  const int m0 = wv * 4 + (lane >> 4), c0 = (int)blockIdx.y * 128 + (lane & 15) * 8;
   if (m0 >= p.M) return;  // uniform over the 16 lanes of a token group
   const u32x4* wq = (const u32x4*)(p.conv_w + (size_t)c0 * 4);
   u32x4* ring = (u32x4*)(p.conv_ring + (size_t)c0 * 4);
   const u32x4 wv4[4] = {wq[0], wq[1], wq[2], wq[3]};
-  u32x4 x[T + 3];  // x[j]: token m0 - 3 + j
+  u32x4 x[4];  // x[j]: token m0 - 3 + j
 #pragma unroll
-  for (int j = 0; j < T + 3; ++j) {
+  for (int j = 0; j < 4; ++j) {
     const int t = min(max(m0 - 3 + j, 0), p.M - 1);
     x[j] = *(const u32x4*)(p.mixed + (size_t)t * p.C + c0);
   }
@@ -959,44 +960,40 @@ __global__ __launch_bounds__(256) void gdn_front_kernel(QhGdnPrepParams p) {
   const bool is_qk = (int)blockIdx.y < 2 * p.Hk;
   uint16_t* ndst = (int)blockIdx.y < p.Hk ? p.qn : p.kn;
   const int kh = (int)blockIdx.y % p.Hk;
+  u32x4 out;
+  float ss = 0.0f, r[8];
 #pragma unroll
-  for (int k = 0; k < T; ++k) {
-    const int m = m0 + k;
-    u32x4 out;
-    float ss = 0.0f, r[8];
+  for (int q = 0; q < 4; ++q) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int e = 4 * (2 * q + h);  // tap j of channel 2 q + h is element e + j of the 32
-        auto wt = [&](int j) {
-          const uint32_t word = wv4[(e + j) >> 3][((e + j) >> 1) & 3];
-          return (j & 1) ? bf_hi(word) : bf_lo(word);
-        };
-        auto xv = [&](int d) { return h ? bf_hi(x[k + 3 - d][q]) : bf_lo(x[k + 3 - d][q]); };
-        float acc = wt(3) * xv(0);
-        acc = fmaf(wt(2), xv(1), acc);
-        acc = fmaf(wt(1), xv(2), acc);
-        acc = fmaf(wt(0), xv(3), acc);
-        r[2 * q + h] = rbf(acc);
-      }
+    for (int h = 0; h < 2; ++h) {
+      const int e = 4 * (2 * q + h);  // tap j of channel 2 q + h is element e + j of the 32
+      auto wt = [&](int j) {
+        const uint32_t word = wv4[(e + j) >> 3][((e + j) >> 1) & 3];
+        return (j & 1) ? bf_hi(word) : bf_lo(word);
+      };
+      auto xv = [&](int d) { return h ? bf_hi(x[3 - d][q]) : bf_lo(x[3 - d][q]); };
+      float acc = wt(3) * xv(0);
+      acc = fmaf(wt(2), xv(1), acc);
+      acc = fmaf(wt(1), xv(2), acc);
+      acc = fmaf(wt(0), xv(3), acc);
+      r[2 * q + h] = rbf(acc);
     }
-    qh_silu_bf(r);
+  }
+  qh_silu_bf(r);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      out[q] = pack_bf2(r[2 * q], r[2 * q + 1]);
-      const float y0 = bf_lo(out[q]), y1 = bf_hi(out[q]);
-      ss += rbf(y0 * y0) + rbf(y1 * y1);
-    }
-    if (m < p.M) *(u32x4*)(p.y + (size_t)m * p.C + c0) = out;
-    if (is_qk) {
-      ss = column_sum<16>(ss);
-      const float inv = rbf(rsqrtf(rbf(rbf(ss) + 1e-6f)));
-      u32x4 nv;
+  for (int q = 0; q < 4; ++q) {
+    out[q] = pack_bf2(r[2 * q], r[2 * q + 1]);
+    const float y0 = bf_lo(out[q]), y1 = bf_hi(out[q]);
+    ss += rbf(y0 * y0) + rbf(y1 * y1);
+  }
+  *(u32x4*)(p.y + (size_t)m0 * p.C + c0) = out;
+  if (is_qk) {
+    ss = column_sum<16>(ss);
+    const float inv = rbf(rsqrtf(rbf(rbf(ss) + 1e-6f)));
+    u32x4 nv;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) nv[q] = pack_bf2(bf_lo(out[q]) * inv, bf_hi(out[q]) * inv);
-      if (m < p.M) *(u32x4*)(ndst + ((size_t)m * p.Hk + kh) * 128 + (lane & 15) * 8) = nv;
-    }
+    for (int q = 0; q < 4; ++q) nv[q] = pack_bf2(bf_lo(out[q]) * inv, bf_hi(out[q]) * inv);
+    *(u32x4*)(ndst + ((size_t)m0 * p.Hk + kh) * 128 + (lane & 15) * 8) = nv;
   }
   if (m0 == 0) {  // the ring's last four positions (older slots of a short prompt stay)
 #pragma unroll
@@ -1267,17 +1264,13 @@ int qh_launch_gdn_prep(const QhGdnPrepParams& p, hipStream_t st) {
     return -1;
   }
   if (p.M <= 0) return 0;
-  // One pass when every row can be moved in 16-byte pieces: 8 tokens per thread
-  // from 512 tokens, 1 below (the threads of a short prompt are its
-  // parallelism).
+  // one pass when every row can be moved in 16-byte pieces
   const void* al[] = {p.mixed, p.y, p.conv_w, p.conv_ring, p.qn, p.kn};
   bool aligned = true;
   for (const void* q : al) aligned = aligned && (uintptr_t)q % 16 == 0;
   if (aligned) {
-    const int T = p.M >= 512 ? 8 : 1;
-    const dim3 grid((unsigned)((p.M + 16 * T - 1) / (16 * T)), (unsigned)(p.C / 128 + 1));
-    if (T == 8) hipLaunchKernelGGL(gdn_front_kernel<8>, grid, dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(gdn_front_kernel<1>, grid, dim3(256), 0, st, p);
+    const dim3 grid((unsigned)(((size_t)p.M + 15) / 16), (unsigned)(p.C / 128 + 1));
+    hipLaunchKernelGGL(gdn_front_kernel, grid, dim3(256), 0, st, p);
     return 0;
   }
   const size_t n = (size_t)p.M * p.C;

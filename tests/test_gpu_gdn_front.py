@@ -33,8 +33,7 @@ def front(mixed, ring, conv_w, a, b, A_log, dt_bias, Hk, Hv, past, off=None):
     return [t.cpu() for t in (y, qn, kn, g, beta, d[1])]
 
 
-# 1 token per thread (16 per block) below 512 tokens, 8 (128 per block) from there; the ring holds
-# the last four positions, so prompts of fewer than 4 tokens keep some of its old ones.
+# 1 token per thread, 16 per block; the ring holds the last four positions, so prompts of fewer than 4 tokens keep some of its old ones.
 # With one buffer 2 bytes past a 16-byte boundary the conv and the norm run as two kernels.
 @pytest.mark.parametrize("M,past,off", [(1, 0, None), (1, 6, None), (2, 3, None), (3, 9, None), (4, 1, None),
                                         (5, 2, None), (31, 0, None), (33, 7, None), (511, 5, None), (512, 0, None),
@@ -68,7 +67,7 @@ def test_gdn_front(M, past, off):
     assert torch.equal(r2, want)
 
 
-@pytest.mark.parametrize("M", [176, 683])   # both thread shapes
+@pytest.mark.parametrize("M", [176, 683])
 def test_conv_silu_every_argument(M):
     """Every finite bf16 value through a conv that passes its newest token: rounded as 64-bit SiLU at
     least as often as fp32 arithmetic is, and never more than one bf16 step off; infinities."""
